@@ -301,12 +301,17 @@ def canary_add_offset(inp: torch.Tensor, offset: int) -> torch.Tensor:
 
 
 def gram(x: torch.Tensor, ws: Optional[Workspace] = None) -> torch.Tensor:
-    """XᵀX per batch, (B, D, D) fp32."""
+    """XᵀX per batch, (B, D, D) fp32.  A tied problem's workspace is carved by
+    that problem's own plan (its K included): carved for another K, the partial
+    sums would land on sub-buffers the EM iteration keeps, its status words
+    among them."""
     require_hip()
     x = _device_tensor(x, "x", torch.float32)
     B, N, D = x.shape
     prob = problem("tied", x.dtype, B, N, D, 1)
     ws = ws or Workspace(prob, x.device)
+    if (ws.prob.covariance_type, ws.prob.B, ws.prob.N, ws.prob.D) == (prob.covariance_type, B, N, D):
+        prob = ws.prob
     out = torch.empty((B, D, D), dtype=torch.float32, device=x.device)
     _check(_lib.gmmxx_hip_gram(ctypes.byref(prob), _ptr(x), _ptr(out), ws.ptr, ws.nbytes, _stream(x.device)),
            "gmmxx_hip_gram")

@@ -237,3 +237,22 @@ def test_tied_jitter_ladder_indefinite_covariance(hip, d):
     _close(m_d, e_m)
     _close(c_d, e_c)
     _close(w_d, e_w)
+
+
+@pytest.mark.parametrize("n,d,k", [(8881, 11, 3), (300, 16, 2), (40000, 64, 8)])
+def test_tied_fit_shares_its_workspace_with_the_gram(hip, n, d, k):
+    """XᵀX and the EM iterations run on one workspace: the gram's partial sums must
+    stay off the iteration's status words (a fit that finds them nonzero raises)."""
+    print(f"[edges] tied gram workspace N={n} D={d} K={k}", flush=True)
+    x, means, covs, w = make_problem("tied", 1, n, d, k, seed=67)
+    prob = hip.problem("tied", torch.float32, 1, n, d, k)
+    ws = hip.Workspace(prob, torch.device(DEV))
+    hip.gram(to_dev(x), ws)
+    assert int(hip.take_status(ws).item()) == 0
+    _, m, c, wt, _ = em.fit(to_dev(x), k, "tied", max_iters=2, tol=0.0, init_means=means, init_covs=covs,
+                            init_weights=w)
+    _, e_m, e_c, e_w, _ = torch_ref.fit(x, k, "tied", max_iters=2, tol=0.0, init_means=means, init_covs=covs,
+                                        init_weights=w)
+    _close(m, e_m)
+    _close(c, e_c)
+    _close(wt, e_w)
