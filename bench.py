@@ -249,8 +249,8 @@ def single_pass(cfg):
     if cfg["cov"] == "spherical" and cfg["dtype"] == "bf16":
         if cfg["D"] <= 64 and cfg["K"] <= 64:
             return "sph_bf16_fused_kernel"
-        if cfg["D"] == 128 and 256 < cfg["K"] <= 1024 and os.environ.get("GMMXX_HIP_NO_COOP") != "1":
-            return "sph_bf16_coop_kernel"
+        if cfg["K"] <= 1024 and os.environ.get("GMMXX_HIP_NO_COOP") != "1":
+            return "sph_bf16_coop_kernel" if cfg["K"] > 256 else "sph_bf16_one_kernel"
         return None
     if cfg["cov"] == "full" and cfg["D"] > 16:
         return None   # whitening E-step, then the statistics kernel

@@ -47,11 +47,12 @@ struct Plan {
   int DP = 0, EP = 0, JP = 0, nk_col = 0, sq_col = 0, sq_n = 0, CW = 0, nw = 0, ktiles = 0, slices = 0, cblocks = 0;
   int lnw = 0, lktiles = 0;  // waves / component tiles of the plain log-normaliser pass (MODE_LSE)
   bool fused = false;        // EM iteration as one fused pass (small K; em_fused.hip)
-  bool coop = false;         // EM iteration as one cooperative pass (spherical bf16, D = 128; em_coop.hip)
+  bool coop = false;         // EM iteration as one cooperative pass (spherical bf16; em_coop.hip)
   bool single = false;       // EM iteration as one tile pass (fp32 x, all K in one workgroup; MODE_STATS_LSE)
   bool xch = false;          // EM iteration as one tile pass whose 2..4 component tiles exchange row partials
   int xslices = 0;           // xch: row slices per batch (grid xslices·ktiles x B, all resident)
   int64_t xrows = 0;         // xch: rows per slice
+  int cDP = 0, cnw = 0;      // coop: padded row width, waves per workgroup
   int cG = 0, cNG = 0, cspb = 0;   // coop: workgroups per group, groups, row items per batch
   int64_t crows = 0;         // coop: rows per item
   int fslices = 0;           // fused: one wave per row slice
@@ -173,19 +174,33 @@ int plan_problem(const gmmxx_problem* p, Plan* pl) {
     q.fslices = (int)((q.N + q.frows - 1) / q.frows);
     q.fparts = (q.fslices + kFusedWaves - 1) / kFusedWaves;
   }
-  // Cooperative single pass: spherical bf16 at D = 128 with 256 < K <= 1024
-  // (groups of 2..4 workgroups; at one group member and at eight the two-pass
-  // kernels measured faster).  Group members must be co-resident, so the grid is
-  // the device's resident capacity rounded to whole groups (multiples of 8
-  // groups keep each group on one XCD).  GMMXX_HIP_NO_COOP=1 selects the
-  // two-pass kernels instead.
+  // Single pass, spherical bf16 with K <= 1024 beyond the fused pass's range: one
+  // workgroup holding every component (K <= 256, em_one.hip), or a group of 2..4
+  // per row slice (em_coop.hip; at eight members the two-pass kernels measured
+  // faster).  N = 1M, two passes -> single pass: D = 64, K = 1000 0.95 -> 0.66-0.70
+  // ms, D = 32, K = 1000 0.83 -> 0.60-0.66, D = 47, K = 324 0.64 -> 0.38; N = 2M,
+  // D = 121, K = 700 5.4 -> 1.76; N = 60000, D = 96, K = 300 0.115 -> 0.064 (widths
+  // other than 32, 64 and 128 were loaded by element).  Group members must
+  // be co-resident, so the grid is the device's resident capacity rounded to
+  // whole groups (multiples of 8 groups keep each group on one XCD).
+  // GMMXX_HIP_NO_COOP=1 selects the two-pass kernels instead.
   const char* no_coop = getenv("GMMXX_HIP_NO_COOP");
-  q.coop = sph_bf && q.DP == 128 && q.D == 128 && q.K > kCoopComps && q.K <= kCoopComps * kMaxCoopGroup &&
-           !(no_coop && no_coop[0] == '1');
+  q.coop = sph_bf && !q.fused && q.K <= kCoopComps * kMaxCoopGroup && !(no_coop && no_coop[0] == '1');
   if (q.coop) {
+    q.cDP = round_up(std::max(q.D, 1), 32);
     q.cG = (q.K + kCoopComps - 1) / kCoopComps;
-    int ng = coop_capacity() / q.cG;
-    if (ng >= 8) ng -= ng % 8;
+    // Waves of one workgroup (32 components each).  At K <= 64 two waves up to 96
+    // columns (N = 1M, D = 96, K = 50: 0.114 against 0.146 ms with four), four
+    // beyond, where two spend longer loading the rows than four on padding
+    // components (D = 121, K = 16: 0.180 against 0.247 ms).
+    q.cnw = q.K <= 64 && q.cDP <= 96 ? 2 : (q.K <= 128 ? 4 : 8);
+    int ng;
+    if (q.cG == 1) {
+      ng = kTargetWaves / q.cnw;   // one round at two resident waves per SIMD
+    } else {
+      ng = coop_capacity(q.cDP, q.cG, q.D == 128) / q.cG;
+      if (ng >= 8) ng -= ng % 8;
+    }
     q.cNG = ng;
     q.coop = ng >= 1;
   }
@@ -254,7 +269,8 @@ int plan_problem(const gmmxx_problem* p, Plan* pl) {
   q.o_waug = take(sph_bf ? BK * 32 * 2 : 0);
   q.o_wmu = take((q.coop || q.fused) ? BK * q.DP * 2 : 0);
   q.o_wsc = take((q.coop || q.fused) ? BK * 4 : 0);
-  q.o_waugs = take(q.fused ? BK * 16 * 2 : 0);
+  const bool one_group = q.fused || (q.coop && q.cG == 1);   // logits as s·(x·μ - ‖x‖²/2 + C')
+  q.o_waugs = take(one_group ? BK * 16 * 2 : 0);
   q.o_cconst = take(BK * 16);
   q.o_covs_used = take(q.cov == SPH ? BK * 4 : (q.cov == DIAG ? BK * q.D * 4 : 0));
   q.o_rowq = take(q.cov == TIED ? BN * 4 : 0);
@@ -267,7 +283,7 @@ int plan_problem(const gmmxx_problem* p, Plan* pl) {
   q.o_stats = take(BK * q.JP * 4);
   // (+B: the tied EM iteration's per-batch log-likelihood shift, after the row partials)
   q.o_ll = take((size_t)q.B * (std::max({q.cblocks, q.fslices, q.cspb, q.slices, q.xslices, q.fw_eblk}) + q.D + 1) * 8);
-  q.o_xch = take(q.coop ? (size_t)q.cNG * kRing * q.cG * kBN * 8
+  q.o_xch = take(q.coop && q.cG > 1 ? (size_t)q.cNG * kRing * q.cG * kBN * 8
                         : (q.xch ? (size_t)q.B * q.xslices * kRing * q.ktiles * kBN * 8 : 0));
   // [0] status of the last cooperative pass (zeroed by its launcher), [1] sticky
   // status since the last gmmxx_hip_take_status
@@ -356,11 +372,12 @@ int run_fused(const Plan& pl, const TileArgs& t, hipStream_t s) {
 }
 // Cooperative single pass: partial statistics per row item and partial log-likelihoods.
 int run_coop(const Plan& pl, const void* x, void* ws, hipStream_t s) {
-  if ((uintptr_t)x % 16 != 0)
+  if (pl.D == 128 && pl.cG > 1 && (uintptr_t)x % 16 != 0)
     return fail(GMMXX_ERR_INVALID_ARGUMENT, "x must be 16-byte aligned for spherical bf16 at D = 128");
   CoopArgs c{};
   c.x = x;
-  c.vec_ok = 1;
+  c.vec = pl.D % 8 == 0 && (uintptr_t)x % 16 == 0;
+  c.DL = pl.DP;
   c.N = pl.N;
   c.D = pl.D;
   c.K = pl.K;
@@ -368,6 +385,7 @@ int run_coop(const Plan& pl, const void* x, void* ws, hipStream_t s) {
   c.w_mu = at<void>(ws, pl.o_wmu);
   c.w_scale = at<float>(ws, pl.o_wsc);
   c.w_aug = at<void>(ws, pl.o_waug);
+  c.w_augs = at<void>(ws, pl.o_waugs);
   c.G = pl.cG;
   c.NG = pl.cNG;
   c.spb = pl.cspb;
@@ -380,7 +398,7 @@ int run_coop(const Plan& pl, const void* x, void* ws, hipStream_t s) {
   // it (a negative value gives up at the first wait: the timeout path, on demand).
   c.spin_limit = 1 << 20;
   if (const char* sl = getenv("GMMXX_HIP_COOP_SPIN_LIMIT")) c.spin_limit = atoi(sl);
-  const int rc = launch_sph_bf16_coop(pl.DP, c, s);
+  const int rc = pl.cG == 1 ? launch_sph_bf16_one(pl.cDP, pl.cnw, c, s) : launch_sph_bf16_coop(pl.cDP, c, s);
   if (rc == -2) return fail(GMMXX_ERR_HIP, "launch of the single-pass cooperative kernel failed");
   if (rc != 0) return fail(GMMXX_ERR_UNSUPPORTED, "no single-pass cooperative kernel for this shape and device");
   return check_hip("cooperative single-pass kernel");
@@ -412,7 +430,7 @@ LlFold ll_fold(const Plan& pl, void* ws, int parts, double inv_total, float* out
   ll.count = parts;
   ll.inv_total = inv_total;
   ll.out = out;
-  if (pl.coop || pl.xch) {
+  if ((pl.coop && pl.cG > 1) || pl.xch) {
     ll.status = at<unsigned>(ws, pl.o_flags);
     ll.sticky = at<unsigned>(ws, pl.o_flags) + 1;
   }
@@ -553,7 +571,7 @@ int prepare(const Plan& pl, const void* x, const float* means, const float* covs
   a.w_aug = (pl.bf && pl.cov == SPH) ? at<void>(ws, pl.o_waug) : nullptr;
   a.w_mu = (pl.coop || pl.fused) ? at<void>(ws, pl.o_wmu) : nullptr;
   a.w_scale = (pl.coop || pl.fused) ? at<float>(ws, pl.o_wsc) : nullptr;
-  a.w_augs = pl.fused ? at<void>(ws, pl.o_waugs) : nullptr;
+  a.w_augs = (pl.fused || (pl.coop && pl.cG == 1)) ? at<void>(ws, pl.o_waugs) : nullptr;
   a.cconst = at<float4>(ws, pl.o_cconst);
   a.gram = shift ? gram : nullptr;
   a.shift = gram ? shift : nullptr;
@@ -715,7 +733,7 @@ int gmmxx_hip_device_info(int device, gmmxx_dev_info* out) {
   int cur = 0;
   if (hipGetDevice(&cur) != hipSuccess) return check_hip("hipGetDevice");
   if (cur != device && hipSetDevice(device) != hipSuccess) return check_hip("hipSetDevice");
-  out->coop_capacity = coop_capacity();
+  out->coop_capacity = coop_capacity(128, kMaxCoopGroup, true);
   if (cur != device && hipSetDevice(cur) != hipSuccess) return check_hip("hipSetDevice");
   return GMMXX_OK;
 }
@@ -813,7 +831,7 @@ int gmmxx_hip_em_phase(const gmmxx_problem* p, int phase, const void* x, float* 
     case GMMXX_PHASE_FINALIZE:
       // A cooperative pass that timed out leaves the parameters as they were.
       finalize(pl, ws, gram, reg_covar, min_weight, pl.N, means, covs, weights, s,
-               (pl.coop || pl.xch) ? coop_status(pl, ws) : nullptr);
+               ((pl.coop && pl.cG > 1) || pl.xch) ? coop_status(pl, ws) : nullptr);
       return check_hip("finalize");
     default:
       return fail(GMMXX_ERR_INVALID_ARGUMENT, "unknown phase");

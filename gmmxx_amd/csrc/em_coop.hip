@@ -1,4 +1,4 @@
-// Single-pass spherical bf16 EM tile for many components at D = 128.
+// Single-pass spherical bf16 EM tile for many components (256 < K <= 1024, D <= 128).
 //
 // The two-pass tile design (em_sph_bf16.hip) computes every logit twice: once
 // for the row log-normalisers and once more for the responsibilities, because
@@ -63,84 +63,16 @@
 
 #include "common.hpp"
 #include "engine.hpp"
+#include "sph_bf16.hpp"
 
 namespace gx {
 
 namespace {
 
-constexpr int kAug = 32;           // augmented k-chunk width (bf16 columns)
-constexpr float kHuge = 1e30f;     // "minus infinity" that stays finite through MFMA
+using namespace sphb;
+
 constexpr int kNW = 8;             // waves per workgroup
-constexpr int kCW = 32;            // components per wave
 constexpr int kNB = 5;             // staged row blocks: i-2 .. i+2
-constexpr int kRS = 48;            // r row stride (bf16): 32 components + padding
-
-typedef short v4s __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-__device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-
-template <typename T>
-__device__ __forceinline__ T ld16(const void* p) { return *reinterpret_cast<const T*>(p); }
-
-template <int CTRL>
-__device__ __forceinline__ float dpp(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
-}
-
-// Sum over groups of G consecutive lanes (G <= 16), result in every lane.
-template <int G>
-__device__ __forceinline__ float group_sum(float v) {
-  if constexpr (G >= 2) v += dpp<0xB1>(v);    // lane ^ 1
-  if constexpr (G >= 4) v += dpp<0x4E>(v);    // lane ^ 2
-  if constexpr (G >= 8) v += dpp<0x141>(v);   // row_half_mirror
-  if constexpr (G >= 16) v += dpp<0x140>(v);  // row_mirror
-  return v;
-}
-
-// v combined with lane l ^ 16 (OFF = 16) or l ^ 32 (OFF = 32).
-template <int OFF, bool MAX>
-__device__ __forceinline__ float lanes_op(float v) {
-  const auto t = (OFF == 16) ? __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false)
-                             : __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  const float a = __uint_as_float(t[0]), b = __uint_as_float(t[1]);
-  return MAX ? fmaxf(a, b) : a + b;
-}
-
-__device__ __forceinline__ void split3(float v, __bf16& h, __bf16& m, __bf16& l) {
-  h = (__bf16)v;
-  const float r = v - (float)h;
-  m = (__bf16)r;
-  l = (__bf16)(r - (float)m);
-}
-
-__device__ __forceinline__ uint32_t pack2(__bf16 a, __bf16 b) {
-  return (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
-}
-
-// Two floats rounded to bf16 (nearest even) in one dword, a in the low half.
-__device__ __forceinline__ uint32_t cvt2(float a, float b) {
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
-}
-
-// Transposing LDS read: in each 16-lane group, lane L supplies the address of
-// an 8-byte chunk; lane i receives word (i % 4) of the chunks of lanes 4j + i/4.
-__device__ __forceinline__ v4s tr16(const __bf16* p) {
-  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)p);
-}
-
-__device__ __forceinline__ bf16x8 cat(v4s lo, v4s hi) {
-  return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-}
-
-// r rows: the 4-element column chunk is XOR-swizzled by (row / 4) % 4, so that
-// 16 lanes writing one chunk of consecutive rows, and the transposing reads of
-// 4 rows x 4 chunks, touch distinct bank pairs.
-__device__ __forceinline__ int rswz(int row, int col) { return col ^ (((row >> 2) & 3) << 2); }
 
 // Exchange slots start with the odd round tag in the high (S) half of every
 // 64-bit word, so no slot reads as a round-0 word before it is written.
@@ -152,17 +84,19 @@ __global__ void coop_zero_kernel(unsigned* p, int n, unsigned* status) {
 
 }  // namespace
 
-// KG: largest group size the instance handles (G <= KG); the partners' words of
-// a block are loaded together into KG registers.
-template <int DP, int KG>
+// DP: row width, padded (the columns past D are staged as zeros).  KG: largest
+// group size the instance handles (G <= KG); the partners' words of a block are
+// loaded together into KG registers.  EXACT: D == DP and 16-byte aligned rows;
+// otherwise rows of any D (a.vec: whole aligned 16-byte chunks).
+template <int DP, int KG, bool EXACT>
 __global__ __launch_bounds__(64 * kNW) void sph_bf16_coop_kernel(CoopArgs a) {
   constexpr int XK = DP / 16;                    // 16-deep k-steps over the x columns (E-GEMM)
   constexpr int XT = DP / 32;                    // 32-wide x tiles of ψ (M-GEMM)
-  constexpr int XS = 176;                        // staged row stride (bf16)
+  constexpr int XS = row_stride(DP);             // staged row stride (bf16)
   static_assert(DP + kAug <= XS, "row does not fit the staging stride");
-  constexpr int JP = DP + 16;                    // statistics columns: x | augmented 0..15
-  constexpr int CPR = DP / 8;                    // 16-byte chunks per row
-  constexpr int NCH = kBN * CPR;                 // chunks per row block
+  constexpr int CPR = row_lanes(DP);             // loading lanes (16-byte chunks) per row
+  static_assert(CPR * 8 >= DP, "a row's chunks cover it");
+  constexpr int NCH = kBN * CPR;                 // chunk slots per row block (DP = 96 leaves 4 of 16 idle)
   constexpr int NTHR = 64 * kNW;
   constexpr int PF = (NCH + NTHR - 1) / NTHR;
   constexpr int RR = kBN + 1;                    // red_* stride per wave
@@ -179,6 +113,7 @@ __global__ __launch_bounds__(64 * kNW) void sph_bf16_coop_kernel(CoopArgs a) {
   const int lr = lane % 32, hf = lane / 32;     // 32x32 MFMA: row / component of a tile, k half
   const int64_t N = a.N;
   const int K = a.K, G = a.G;
+  const int DL = EXACT ? DP : a.DL;             // columns of w_mu; statistics rows are DL + 16 wide
 
   // Group and member: groups on one XCD (ids congruent mod 8) when NG % 8 == 0.
   const int id = blockIdx.x;
@@ -235,7 +170,7 @@ __global__ __launch_bounds__(64 * kNW) void sph_bf16_coop_kernel(CoopArgs a) {
         const size_t bk = (size_t)b * K + kk;
 #pragma unroll
         for (int t = 0; t < XK; ++t)
-          wmu[t] = ld16<bf16x8>(reinterpret_cast<const __bf16*>(a.w_mu) + bk * DP + 16 * t + 8 * hf);
+          wmu[t] = ld16<bf16x8>(reinterpret_cast<const __bf16*>(a.w_mu) + bk * DL + 16 * t + 8 * hf);
         waug = ld16<bf16x8>(reinterpret_cast<const __bf16*>(a.w_aug) + bk * kAug + 8 * hf);
       } else {
 #pragma unroll
@@ -259,14 +194,19 @@ __global__ __launch_bounds__(64 * kNW) void sph_bf16_coop_kernel(CoopArgs a) {
     // x rows of this item, addressed with 32-bit offsets from a uniform base (the
     // launcher keeps an item under 2^31 bytes).  Rows past the item end read the
     // last valid row (in bounds, no branch) and are zeroed.
-    const __bf16* xi = reinterpret_cast<const __bf16*>(a.x) + ((size_t)b * N + rbeg) * DP;
+    const int D = EXACT ? DP : a.D;
+    const __bf16* xi = reinterpret_cast<const __bf16*>(a.x) + ((size_t)b * N + rbeg) * D;
     const int nrows = (int)(rend - rbeg);
     uint4 pf[PF];
     auto load_chunk = [&](int c, int r0) -> uint4 {
       const int r = r0 + c / CPR, cc = (c % CPR) * 8;
       const bool valid = r < nrows;
-      const uint4 v = *reinterpret_cast<const uint4*>(xi + (valid ? r : nrows - 1) * DP + cc);
-      return valid ? v : make_uint4(0, 0, 0, 0);
+      if constexpr (EXACT) {
+        const uint4 v = *reinterpret_cast<const uint4*>(xi + (valid ? r : nrows - 1) * DP + cc);
+        return valid ? v : make_uint4(0, 0, 0, 0);
+      } else {
+        return load_row_chunk<false>(xi + (valid ? r : nrows - 1) * D, cc, D, a.vec, valid);
+      }
     };
     auto fetch = [&](int r0) {
 #pragma unroll
@@ -285,7 +225,7 @@ __global__ __launch_bounds__(64 * kNW) void sph_bf16_coop_kernel(CoopArgs a) {
           const int r = c / CPR, cc = c % CPR;
           const uint4 raw = pf[i];
           __bf16* row = xs + buf * kBN * XS + r * XS;
-          *reinterpret_cast<uint4*>(row + 8 * cc) = raw;
+          if (8 * CPR == DP || 8 * cc < DP) *reinterpret_cast<uint4*>(row + 8 * cc) = raw;
           const uint32_t w4[4] = {raw.x, raw.y, raw.z, raw.w};
           float q = 0.f;
 #pragma unroll
@@ -483,11 +423,11 @@ __global__ __launch_bounds__(64 * kNW) void sph_bf16_coop_kernel(CoopArgs a) {
         // the transcendental unit then works while the matrix core does
         // (measured 2 % faster per C2 pass than after the M-GEMM).
         const float m = row_max(T);
+        constexpr int HK = 2 * (XT + 1) < 8 ? 2 * (XT + 1) : 8, PH = (16 + HK - 1) / HK;   // MFMAs with, exps per MFMA
         mgemm((i + kNB - 2) % kNB, [&](int k) {
-          if (k < 8) {
-            er[PB][2 * k] = fast_exp2(T[2 * k] - m);
-            er[PB][2 * k + 1] = fast_exp2(T[2 * k + 1] - m);
-          }
+#pragma unroll
+          for (int u = 0; u < PH; ++u)
+            if (PH * k + u < 16) er[PB][PH * k + u] = fast_exp2(T[PH * k + u] - m);
         });
         lse_sums(m, PB_);
       }
@@ -563,10 +503,12 @@ __global__ __launch_bounds__(64 * kNW) void sph_bf16_coop_kernel(CoopArgs a) {
     for (int v = 0; v < 16; ++v) {
       const int kk = kbase + 8 * (v / 4) + 4 * hf + (v % 4);
       if (kk < K) {
-        float* dst = a.part_stats + (((size_t)sl * a.B + b) * K + kk) * JP;
+        // statistics row of width DL + 16: x | augmented 0..15 (DL > DP: zeros between)
+        float* dst = a.part_stats + (((size_t)sl * a.B + b) * K + kk) * (DL + 16);
 #pragma unroll
         for (int xt = 0; xt < XT; ++xt) dst[32 * xt + lr] = accx[xt][v];
-        if (lr < 16) dst[DP + lr] = acca[v];
+        if (!EXACT && DP == 96) dst[DP + lr] = 0.f;
+        if (lr < 16) dst[DL + lr] = acca[v];
       }
     }
     if (mem == 0 && wave == 0) {
@@ -576,42 +518,65 @@ __global__ __launch_bounds__(64 * kNW) void sph_bf16_coop_kernel(CoopArgs a) {
   }
 }
 
-int coop_capacity() {
-  // Resident workgroups of the kernel on the current device (cached per device;
-  // concurrent first calls store the same value); 256 when no device is visible
-  // (workspace sizing on a machine without a GPU).
-  static std::atomic<int> cache[64] = {};
+namespace {
+
+// The instance for a padded width, group size and row alignment.
+template <int DP, bool EXACT>
+const void* coop_fn_dp(int G) {
+  return G <= 2 ? reinterpret_cast<const void*>(sph_bf16_coop_kernel<DP, 2, EXACT>)
+                : reinterpret_cast<const void*>(sph_bf16_coop_kernel<DP, 4, EXACT>);
+}
+const void* coop_fn(int dp, int G, bool exact) {
+  switch (dp) {
+    case 32: return coop_fn_dp<32, false>(G);
+    case 64: return coop_fn_dp<64, false>(G);
+    case 96: return coop_fn_dp<96, false>(G);
+    case 128: return exact ? coop_fn_dp<128, true>(G) : coop_fn_dp<128, false>(G);
+    default: return nullptr;
+  }
+}
+
+}  // namespace
+
+int coop_capacity(int dp, int G, bool exact) {
+  // Resident workgroups of the instance on the current device (cached per device
+  // and instance; concurrent first calls store the same value); 256 when no device
+  // is visible (workspace sizing on a machine without a GPU).
+  static std::atomic<int> cache[64][4][2][2] = {};
   int ndev = 0, dev = 0;
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0 || hipGetDevice(&dev) != hipSuccess || dev >= 64) {
     (void)hipGetLastError();
     return 256;
   }
-  const int cached = cache[dev].load(std::memory_order_relaxed);
+  const void* fn = coop_fn(dp, G, exact);
+  if (!fn) return 0;
+  std::atomic<int>& c = cache[dev][dp / 32 - 1][G > 2][exact];
+  const int cached = c.load(std::memory_order_relaxed);
   if (cached > 0) return cached;
   int cus = 0, per = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, sph_bf16_coop_kernel<128, 4>, 64 * kNW, 0) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, fn, 64 * kNW, 0) != hipSuccess ||
       cus <= 0 || per <= 0) {
     (void)hipGetLastError();
     return 256;
   }
-  cache[dev].store(cus * per, std::memory_order_relaxed);
+  c.store(cus * per, std::memory_order_relaxed);
   return cus * per;
 }
 
 int launch_sph_bf16_coop(int dp, const CoopArgs& a, hipStream_t s) {
-  if (dp != 128 || a.G < 2 || a.G > kMaxCoopGroup) return -1;
+  const bool exact = dp == 128 && a.D == 128 && a.vec;
+  const void* fn = coop_fn(dp, a.G, exact);
+  if (!fn || a.D > dp || a.DL < dp || a.G < 2 || a.G > kMaxCoopGroup) return -1;
   const int grid = a.NG * a.G;
   // The exchange slots (64-bit words) start with the odd round tag, the status word at zero.
   const int nwords = a.NG * kRing * a.G * kBN * 2;
   coop_zero_kernel<<<(nwords + 1 + 255) / 256, 256, 0, s>>>(reinterpret_cast<unsigned*>(a.xch), nwords, a.status);
-  const void* fn = a.G <= 2 ? reinterpret_cast<const void*>(sph_bf16_coop_kernel<128, 2>)
-                            : reinterpret_cast<const void*>(sph_bf16_coop_kernel<128, 4>);
   // A plain launch of at most the resident capacity: on an otherwise idle device
   // every workgroup is dispatched at once.  Nothing else guarantees it, so the
   // bounded waits are the guard: a member that never meets its partners gives
   // up, sets the status word and drains.
-  if (grid > coop_capacity()) return -1;
+  if (grid > coop_capacity(dp, a.G, exact)) return -1;
   CoopArgs args = a;
   void* params[] = {&args};
   const hipError_t e = hipLaunchKernel(fn, dim3(grid), dim3(64 * kNW), params, 0, s);

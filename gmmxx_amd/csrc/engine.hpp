@@ -65,9 +65,10 @@ int launch_sph_bf16(int dp, int nw, int mode, const TileArgs& a, dim3 grid, hipS
 constexpr int kFusedWaves = 4;
 int launch_sph_bf16_fused(int dp, int k, const TileArgs& a, int slices, hipStream_t s);
 
-// Single-pass cooperative kernel (em_coop.hip): spherical bf16 at D = 128 with
-// G = ceil(K / 256) workgroups per group of rows, 2 <= G <= kMaxCoopGroup
-// (256 < K <= 1024, where it measured faster than the two-pass kernels).
+// Single-pass kernels, spherical bf16 at D <= 128, dp in {32, 64, 96, 128}: one
+// workgroup of nw in {2 (dp <= 96), 4, 8} waves holding every component (em_one.hip,
+// K <= 256), or a group of G = ceil(K / 256) workgroups of 8 waves per row slice
+// that exchange row partials (em_coop.hip, 2 <= G <= kMaxCoopGroup, K <= 1024).
 constexpr int kCoopComps = 256;      // components per workgroup
 constexpr int kMaxCoopGroup = 4;
 constexpr int kRing = 4;             // exchange slots per group
@@ -75,12 +76,14 @@ constexpr uint32_t kTagOdd = 0x80000000u;  // round-parity tag bit of an exchang
 
 struct CoopArgs {
   const void* x;               // [B][N][D] bf16
-  int vec_ok;
+  int vec;                     // rows 16-byte aligned (D % 8 == 0 and x 16-byte aligned)
   int64_t N;
   int D, K, B;
-  const void* w_mu;            // [B][K][DP] the means, bf16
+  int DL;                      // columns of w_mu; the statistics rows are DL + 16 wide
+  const void* w_mu;            // [B][K][DL] the means, bf16
   const float* w_scale;        // [B][K] log2(e)/σ²
   const void* w_aug;           // [B][K][32] bf16
+  const void* w_augs;          // [B][K][16] bf16 (em_one.hip; as TileArgs)
   int G;                       // workgroups per group
   int NG;                      // groups (grid = NG * G)
   int spb;                     // row items per batch
@@ -91,9 +94,11 @@ struct CoopArgs {
   unsigned* status;            // nonzero after a timed-out wait (zeroed by the launcher)
   int spin_limit;
 };
-// Resident workgroups of the cooperative kernel on the current device.
-int coop_capacity();
+// Resident workgroups of an instance on the current device (exact: D == dp == 128, aligned rows).
+int coop_capacity(int dp, int G, bool exact);
 int launch_sph_bf16_coop(int dp, const CoopArgs& a, hipStream_t s);
+// (a.G, a.xch and a.status unused; a.NG workgroups)
+int launch_sph_bf16_one(int dp, int nw, const CoopArgs& a, hipStream_t s);
 
 // Full covariance at 16 < D <= 128 (em_full_wide.hip): whitening E-step and
 // weighted-Gram statistics on split-bf16 MFMA operands (the statistics at DP = 128

@@ -113,8 +113,8 @@ int gmmxx_hip_em_step(const gmmxx_problem* p, const void* x, float* means, float
  * when a single pass whose workgroups exchange row partials gave up waiting for
  * a partner workgroup (the members of a group were not all resident: another
  * kernel or process held part of the GPU).  Two passes do this: the cooperative
- * kernel (spherical bf16 at D = 128, 256 < K <= 1024; GMMXX_HIP_NO_COOP=1
- * selects two passes instead) and the exchange pass (fp32 x: spherical at
+ * kernel (spherical bf16, 256 < K <= 1024; GMMXX_HIP_NO_COOP=1 selects two
+ * passes instead) and the exchange pass (fp32 x: spherical at
  * D <= 128, tied and diag at D <= 64, each with 256 < K <= 1024, i.e. two to
  * four component tiles of 256; GMMXX_HIP_NO_XCH=1 selects two passes
  * instead).  Such an iteration writes NaN to its lower bound (or ll_sum) and
