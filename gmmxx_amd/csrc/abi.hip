@@ -581,21 +581,28 @@ int prepare(const Plan& pl, const void* x, const float* means, const float* covs
   return check_hip("parameter preparation");
 }
 
-// Log-normaliser pass: per-k-tile partials, then the per-row combine.
+// Log-normaliser pass: per-k-tile partials, then the per-row combine.  Labels
+// alone take no exponentials (MODE_IDX), no tied row forms (a row constant) and,
+// with one component tile, no combine.
 int lse_pass(const Plan& pl, const void* x, void* ws, float* scores, int64_t* labels, bool with_ll,
              hipStream_t s) {
-  const TileArgs t = tile_args(pl, x, ws);
-  if (run_tile(pl, labels ? MODE_LSE_IDX : MODE_LSE, t, s) != 0)
+  const bool only = labels && !scores && !with_ll;
+  TileArgs t = tile_args(pl, x, ws, /*em=*/only);
+  const bool direct = only && pl.ktiles == 1;
+  if (direct) t.labels = labels;
+  if (run_tile(pl, only ? MODE_IDX : (labels ? MODE_LSE_IDX : MODE_LSE), t, s) != 0)
     return fail(GMMXX_ERR_UNSUPPORTED, "no tile kernel for this shape");
+  if (direct) return check_hip("label pass");
   CombineArgs c{};
   c.B = pl.B;
   c.ktiles = labels ? pl.ktiles : pl.lktiles;
   c.N = pl.N;
   c.part_ms = t.part_ms;
   c.part_idx = t.part_idx;
-  c.lse2 = at<float>(ws, pl.o_lse2);
+  c.lse2 = only ? nullptr : at<float>(ws, pl.o_lse2);
   c.scores = scores;
   c.labels = labels;
+  c.max_only = only;
   c.ll_part = with_ll ? at<double>(ws, pl.o_ll) : nullptr;
   launch_combine(c, s);
   return check_hip("log-normaliser pass");
@@ -993,7 +1000,7 @@ int gmmxx_hip_estep_stats_topk(const gmmxx_problem* p, const void* x, const floa
     // log-normaliser of a single component) and its index; the statistics pass
     // then gives that component r = 1 by index, no logits stored.
     TileArgs t = tile_args(pl, x, ws);
-    if (run_tile(pl, MODE_LSE_IDX, t, s) != 0) return fail(GMMXX_ERR_UNSUPPORTED, "no tile kernel for this shape");
+    if (run_tile(pl, MODE_IDX, t, s) != 0) return fail(GMMXX_ERR_UNSUPPORTED, "no tile kernel for this shape");
     CombineArgs c{};
     c.B = pl.B;
     c.ktiles = pl.ktiles;
@@ -1096,7 +1103,8 @@ int gmmxx_hip_score(const gmmxx_problem* p, const void* x, const float* means, c
   if (!means || !covs || !weights) return fail(GMMXX_ERR_INVALID_ARGUMENT, "NULL parameter buffer");
   const hipStream_t s = (hipStream_t)stream;
   if (pl.w16) return run_w16(pl, x, means, covs, weights, ws, scores, labels, nullptr, s);
-  if ((rc = prepare(pl, x, means, covs, weights, 0.0, 1e-8, 0, ws, s))) return rc;
+  if (!scores && !labels) return GMMXX_OK;
+  if ((rc = prepare(pl, x, means, covs, weights, 0.0, 1e-8, 0, ws, s, /*rowquad=*/scores != nullptr))) return rc;
   if (pl.fw) {
     FwArgs a = fw_args(pl, x, ws);
     a.l2 = nullptr;

@@ -15,11 +15,13 @@ enum Cov { SPH = 0, DIAG = 1, TIED = 2, FULL = 3 };
 // rest zero, against the top-k log-normaliser.
 // MODE_STATS_LSE / MODE_PROBA_LSE: the statistics / responsibility pass with the
 // row log-normalisers formed inside the workgroup (every component is in it).
+// MODE_IDX: MODE_LSE_IDX without the sums (labels or the row maximum alone): no
+// exponentials.
 // MODE_STATS_XCH: the statistics pass with the row log-normalisers merged across
 // the workgroups that hold a row slice's component tiles (exchanged partials).
 enum Mode {
   MODE_LSE = 0, MODE_STATS = 1, MODE_PROBA = 2, MODE_LSE_IDX = 3, MODE_STATS_TOPK = 4, MODE_STATS_LSE = 5,
-  MODE_PROBA_LSE = 6, MODE_STATS_XCH = 7
+  MODE_PROBA_LSE = 6, MODE_STATS_XCH = 7, MODE_IDX = 8
 };
 
 constexpr float kLog2e = 1.4426950408889634f;
@@ -85,6 +87,13 @@ __device__ __forceinline__ float clamp_lo(float v, float lo) { return v < lo ? l
 
 __device__ __forceinline__ float to_f32(float v) { return v; }
 __device__ __forceinline__ float to_f32(__bf16 v) { return (float)v; }
+
+// 16 bytes at an element address of any alignment (one global load instruction).
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ uint4 ld16_any(const void* p) {
+  const u32x4_any v = *reinterpret_cast<const u32x4_any*>(p);
+  return make_uint4(v[0], v[1], v[2], v[3]);
+}
 
 // Merge two (max, scaled-sum, argmax) triples; ties keep the smaller index.
 __device__ __forceinline__ void lse_merge(float& m, float& s, int& idx, float m2, float s2, int i2) {

@@ -99,8 +99,9 @@ __device__ __forceinline__ uint32_t pack2(__bf16 a, __bf16 b) {
 
 template <int DP, int NW, int MODE>
 __global__ __launch_bounds__(64 * NW) void sph_bf16_kernel(TileArgs a) {
-  constexpr bool LSE = (MODE == MODE_LSE || MODE == MODE_LSE_IDX);
-  constexpr bool WANT_IDX = MODE == MODE_LSE_IDX;
+  constexpr bool LSE = (MODE == MODE_LSE || MODE == MODE_LSE_IDX || MODE == MODE_IDX);
+  constexpr bool WANT_IDX = MODE == MODE_LSE_IDX || MODE == MODE_IDX;
+  constexpr bool WANT_SUM = MODE != MODE_IDX;    // (labels or the row maximum alone need no exponentials)
   constexpr bool STATS = MODE == MODE_STATS || MODE == MODE_STATS_TOPK;
   constexpr bool TOPK = MODE == MODE_STATS_TOPK;
   constexpr int CW = 32, CT = 2;                 // components per wave, 16-wide tiles
@@ -129,7 +130,7 @@ __global__ __launch_bounds__(64 * NW) void sph_bf16_kernel(TileArgs a) {
   __shared__ __align__(16) int thri_s[TOPK ? NB * kBN : 4];
   constexpr int RS = kBN + 1;                    // red_* stride per wave (conflict-free reads)
   __shared__ float red_m[LSE ? 2 * NW * RS : 1];   // [parity][wave][row]
-  __shared__ float red_s[LSE ? 2 * NW * RS : 1];
+  __shared__ float red_s[LSE && WANT_SUM ? 2 * NW * RS : 1];
   __shared__ int red_i[WANT_IDX ? 2 * NW * RS : 1];
 
   const int tid = threadIdx.x;
@@ -297,13 +298,16 @@ __global__ __launch_bounds__(64 * NW) void sph_bf16_kernel(TileArgs a) {
       if (tid < kBN * NW) {
         const int r = tid / NW, w = tid % NW;
         const int o = (pb * NW + w) * RS + r;
-        const float mw = red_m[o], sw = red_s[o];
+        const float mw = red_m[o];
         const float M = group_max<NW>(mw);
-        const float t = group_sum<NW>(sw * fast_exp2(mw - M));
+        float t = 0.f;
+        if constexpr (WANT_SUM) t = group_sum<NW>(red_s[o] * fast_exp2(mw - M));
         int idx = 0;
         if constexpr (WANT_IDX) idx = group_min_i<NW>((mw == M) ? red_i[o] : 0x7fffffff);
         const int64_t n = n0 + r;
-        if (w == 0 && n < rend) {
+        if (MODE == MODE_IDX && a.labels) {       // (uniform) every component is in this workgroup
+          if (w == 0 && n < rend) a.labels[(size_t)b * N + n] = (int64_t)idx;
+        } else if (w == 0 && n < rend) {
           const size_t og = ((size_t)ktile * a.B + b) * N + n;
           reinterpret_cast<float2*>(a.part_ms)[og] = make_float2(M, t);
           if constexpr (WANT_IDX) a.part_idx[og] = idx;
@@ -418,15 +422,17 @@ __global__ __launch_bounds__(64 * NW) void sph_bf16_kernel(TileArgs a) {
           idx = lanes_min_i<32>(lanes_min_i<16>(idx));
         }
         float s = 0.f;
+        if constexpr (WANT_SUM) {
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct)
+          for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-          for (int v = 0; v < 4; ++v) s += fast_exp2(A.t[ct][nt][v] - m);
-        s = lanes_op<32, false>(lanes_op<16, false>(s));
+            for (int v = 0; v < 4; ++v) s += fast_exp2(A.t[ct][nt][v] - m);
+          s = lanes_op<32, false>(lanes_op<16, false>(s));
+        }
         if (g == 0) {
           const int o = (pb * NW + wave) * RS + r;
           red_m[o] = m;
-          red_s[o] = s;
+          if constexpr (WANT_SUM) red_s[o] = s;
           if constexpr (WANT_IDX) red_i[o] = idx;
         }
       }
@@ -579,6 +585,7 @@ static int launch_sph_bf16_nw(int mode, const TileArgs& a, dim3 grid, hipStream_
   switch (mode) {
     case MODE_LSE: sph_bf16_kernel<DP, NW, MODE_LSE><<<grid, block, 0, s>>>(a); break;
     case MODE_LSE_IDX: sph_bf16_kernel<DP, NW, MODE_LSE_IDX><<<grid, block, 0, s>>>(a); break;
+    case MODE_IDX: sph_bf16_kernel<DP, NW, MODE_IDX><<<grid, block, 0, s>>>(a); break;
     case MODE_STATS: sph_bf16_kernel<DP, NW, MODE_STATS><<<grid, block, 0, s>>>(a); break;
     case MODE_PROBA: sph_bf16_kernel<DP, NW, MODE_PROBA><<<grid, block, 0, s>>>(a); break;
     case MODE_STATS_TOPK: sph_bf16_kernel<DP, NW, MODE_STATS_TOPK><<<grid, block, 0, s>>>(a); break;

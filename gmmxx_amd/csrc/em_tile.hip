@@ -17,6 +17,9 @@
 //               sum (and, for _IDX, first-index argmax) are reduced across
 //               lanes with two shuffles and across waves through LDS, and
 //               written as one partial per row and component tile.
+//   MODE_IDX    MODE_LSE_IDX for callers of the argmax (or the row maximum) alone:
+//               no exponentials and no sums; with one component tile the labels
+//               are written here and no combine pass runs.
 //   MODE_STATS  E-GEMM in "data rows" orientation (C = φ·Wᵀ); the epilogue turns
 //               logits into responsibilities r = 2^(l2 - lse2) in registers and
 //               feeds them directly as the A operand of the M-GEMM acc += rᵀ·ψ,
@@ -171,11 +174,14 @@ __device__ __forceinline__ void merge_waves(int nw, const float* rm, const float
   }
 }
 
-template <int COV, typename XT, int DP, int CW, int MODE>
+// EX: D == DP, known at compile time (full covariance at D = 16: without the row-tail
+// branches of `settle` the C5 pass measured 1.5 % faster).
+template <int COV, typename XT, int DP, int CW, int MODE, bool EX = false>
 __global__ __launch_bounds__(512) void em_tile_kernel(TileArgs a) {
   constexpr bool BF = sizeof(XT) == 2;
-  constexpr bool LSE = (MODE == MODE_LSE || MODE == MODE_LSE_IDX);
-  constexpr bool WANT_IDX = MODE == MODE_LSE_IDX;
+  constexpr bool LSE = (MODE == MODE_LSE || MODE == MODE_LSE_IDX || MODE == MODE_IDX);
+  constexpr bool WANT_IDX = MODE == MODE_LSE_IDX || MODE == MODE_IDX;
+  constexpr bool WANT_SUM = MODE != MODE_IDX;
   constexpr bool SLSE = MODE == MODE_STATS_LSE || MODE == MODE_PROBA_LSE;
   constexpr bool XCH = MODE == MODE_STATS_XCH;
   constexpr bool STATS = MODE == MODE_STATS || MODE == MODE_STATS_TOPK || MODE == MODE_STATS_LSE || XCH;
@@ -232,7 +238,7 @@ __global__ __launch_bounds__(512) void em_tile_kernel(TileArgs a) {
   __shared__ float thr_s[TOPK ? NB * kBN : 1];     // top-k threshold logit and index per row
   __shared__ int thri_s[TOPK ? NB * kBN : 1];
   __shared__ float red_m[(LSE || SLSE || XCH) ? 2 * kBN * 8 : 1];   // [parity][row][wave]
-  __shared__ float red_s[(LSE || SLSE || XCH) ? 2 * kBN * 8 : 1];
+  __shared__ float red_s[((LSE && WANT_SUM) || SLSE || XCH) ? 2 * kBN * 8 : 1];
   __shared__ __align__(16) float lsw[(SLSE || XCH) ? 8 * kBN : 4];   // [wave][row] merged log-normalisers
   __shared__ int red_i[WANT_IDX ? 2 * kBN * 8 : 1];
 
@@ -243,7 +249,7 @@ __global__ __launch_bounds__(512) void em_tile_kernel(TileArgs a) {
   const int g = lane / 16, li = lane % 16;
   const int b = blockIdx.y;
   const int64_t N = a.N;
-  const int K = a.K, D = a.D;
+  const int K = a.K, D = EX ? DP : a.D;
 
   // XCD-aware block mapping: consecutive logical ids land on one XCD, so the
   // k-tiles that share a row slice are co-scheduled and hit the same L2.
@@ -366,30 +372,65 @@ __global__ __launch_bounds__(512) void em_tile_kernel(TileArgs a) {
 
   // ---- row-block loader ----
   uint4 pf[PF];
-  auto load_chunk = [&](int c, int64_t n0) -> uint4 {
+  // Raw 16 bytes of chunk c of the block at n0 (uniform base, 32-bit offsets): rows
+  // past the slice read its last row, a chunk that passes its row's end the row's
+  // last VEC columns.  `settle` shifts and zeroes when the data is used, so nothing
+  // here waits for the load (shifted in the fetch itself, the wait came there and
+  // the pass lost 5 % to loading by element).  Label pass at N = 1M, D = 100,
+  // K = 500: 0.84 -> 0.65 ms with the exponentials gone too; the 32-bit offsets also
+  // took the C3 exchange pass from 29 spilled VGPRs to 20 (30.9 -> 30.4 ms a fit).
+  auto rows_left = [&](int64_t n0) -> int { return rend - n0 < kBN ? (int)(rend - n0) : kBN; };
+  auto load_chunk = [&](int c, int64_t n0, int left) -> uint4 {
     const int r = c / CPR, cc = (c % CPR) * VEC;
-    const int64_t n = n0 + r;
-    if (n >= rend) return make_uint4(0, 0, 0, 0);
-    if (a.vec_ok) return *reinterpret_cast<const uint4*>(xb + (size_t)n * D + cc);
+    const XT* blk = xb + (size_t)n0 * D;
+    const int row = (r < left ? r : left - 1) * D;
+    return ld16_any(blk + (row + (cc < D - VEC ? cc : D - VEC)));
+  };
+  auto settle = [&](uint4 raw, int cc, int r, int left) -> uint4 {
+    if (D < DP) {                            // (uniform) columns past the row's end are zero
+      if constexpr (!BF) {
+        if (D % VEC && D > VEC) {
+          const int over = cc + VEC - D;     // of this chunk; the load was shifted by as many
+          const int s = over > 0 ? over : 0;
+          if (s & 2) raw = make_uint4(raw.z, raw.w, 0u, 0u);
+          if (s & 1) raw = make_uint4(raw.y, raw.z, raw.w, 0u);
+        }
+      }
+      if (cc >= D) raw = make_uint4(0, 0, 0, 0);
+    }
+    if (left < kBN && r >= left) raw = make_uint4(0, 0, 0, 0);
+    return raw;
+  };
+  // Rows shorter than one load (16 bytes could pass the end of x) are read by element
+  // when they are staged.
+  const bool narrow = DP <= 16 && D < VEC;   // (uniform)
+  auto load_narrow = [&](int c, int64_t n0, int left) -> uint4 {
+    const int r = c / CPR, cc = (c % CPR) * VEC;
+    const XT* row = xb + (size_t)(n0 + (r < left ? r : left - 1)) * D;
     union { uint4 u; XT e[VEC]; } t;
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) t.e[j] = (cc + j < D) ? xb[(size_t)n * D + cc + j] : (XT)0.f;
+    for (int j = 0; j < VEC; ++j) t.e[j] = (r < left && cc + j < D) ? row[cc + j] : (XT)0.f;
     return t.u;
   };
   auto fetch = [&](int64_t n0) {
+    if (narrow) return;
+    const int left = rows_left(n0);
 #pragma unroll
     for (int i = 0; i < PF; ++i) {
       const int c = tid + i * nthr;
-      if (c < NCH) pf[i] = load_chunk(c, n0);
+      if (c < NCH) pf[i] = load_chunk(c, n0, left);
     }
   };
   // Writes the block's staged rows and features into buffer `buf`.
   auto stash = [&](int buf, int64_t n0) {
     int i = 0;
+    const int left = rows_left(n0);
     for (int c = tid; c < NCH; c += nthr, ++i) {          // uniform per wave (NCH % 64 == 0)
-      const uint4 raw = (i < PF) ? pf[i < PF ? i : 0] : load_chunk(c, n0);
       const int r = c / CPR, cc = (c % CPR) * VEC;
       const int64_t n = n0 + r;
+      uint4 raw;
+      if (narrow) raw = load_narrow(c, n0, left);
+      else raw = settle((i < PF) ? pf[i < PF ? i : 0] : load_chunk(c, n0, left), cc, r, left);
       union { uint4 u; XT e[VEC]; } t;
       t.u = raw;
       float v[VEC];
@@ -570,7 +611,7 @@ __global__ __launch_bounds__(512) void em_tile_kernel(TileArgs a) {
     if (tid < kBN * nw) {
       const int r = tid / nw, w = tid % nw;
       const int o = (pb * kBN + r) * 8 + w;
-      const float mw = red_m[o], sw = red_s[o];
+      const float mw = red_m[o];
       float M;
       switch (nw) {
         case 1: M = mw; break;
@@ -578,7 +619,8 @@ __global__ __launch_bounds__(512) void em_tile_kernel(TileArgs a) {
         case 4: M = group_max<4>(mw); break;
         default: M = group_max<8>(mw); break;
       }
-      float t = sw * fast_exp2(mw - M);
+      float t = 0.f;
+      if constexpr (WANT_SUM) t = red_s[o] * fast_exp2(mw - M);
       int idx = 0;
       if constexpr (WANT_IDX) idx = (mw == M) ? red_i[o] : 0x7fffffff;
       switch (nw) {
@@ -588,7 +630,9 @@ __global__ __launch_bounds__(512) void em_tile_kernel(TileArgs a) {
         default: t = group_sum<8>(t); if (WANT_IDX) idx = group_min_i<8>(idx); break;
       }
       const int64_t n = n0 + r;
-      if (w == 0 && n < rend) {
+      if (MODE == MODE_IDX && a.labels) {       // (uniform) every component is in this workgroup
+        if (w == 0 && n < rend) a.labels[(size_t)b * N + n] = (int64_t)idx;
+      } else if (w == 0 && n < rend) {
         const size_t og = ((size_t)ktile * a.B + b) * N + n;
         reinterpret_cast<float2*>(a.part_ms)[og] = make_float2(M, t);
         if constexpr (WANT_IDX) a.part_idx[og] = idx;
@@ -768,16 +812,18 @@ __global__ __launch_bounds__(512) void em_tile_kernel(TileArgs a) {
           idx = (lm == m) ? idx : 0x7fffffff;
           idx = lanes_min_i<32>(lanes_min_i<16>(idx));
         }
-        float s = 0.f;
-#pragma unroll
-        for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-          for (int v = 0; v < 4; ++v) s += fast_exp2(l2v[ct][v] - m);
-        s = lanes_op<32, false>(lanes_op<16, false>(s));
         // Every lane of the row group holds the same values; all write (no branch).
         const int o = (pb * kBN + r) * 8 + wave;
         red_m[o] = m;
-        red_s[o] = s;
+        if constexpr (WANT_SUM) {
+          float s = 0.f;
+#pragma unroll
+          for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) s += fast_exp2(l2v[ct][v] - m);
+          s = lanes_op<32, false>(lanes_op<16, false>(s));
+          red_s[o] = s;
+        }
         if constexpr (WANT_IDX) red_i[o] = idx;
       }
     } else {
@@ -1143,18 +1189,19 @@ __global__ __launch_bounds__(512) void em_tile_kernel(TileArgs a) {
   }
 }
 
-template <int COV, typename XT, int DP>
+template <int COV, typename XT, int DP, bool EX = false>
 static int launch_tile_t(int mode, const TileArgs& a, dim3 grid, int nw, hipStream_t s) {
   constexpr int CW = cw_for<COV, DP, sizeof(XT) == 2>();
   const dim3 block(64 * nw);
   switch (mode) {
-    case MODE_LSE: em_tile_kernel<COV, XT, DP, CW, MODE_LSE><<<grid, block, 0, s>>>(a); break;
-    case MODE_LSE_IDX: em_tile_kernel<COV, XT, DP, CW, MODE_LSE_IDX><<<grid, block, 0, s>>>(a); break;
-    case MODE_STATS: em_tile_kernel<COV, XT, DP, CW, MODE_STATS><<<grid, block, 0, s>>>(a); break;
-    case MODE_PROBA: em_tile_kernel<COV, XT, DP, CW, MODE_PROBA><<<grid, block, 0, s>>>(a); break;
-    case MODE_STATS_TOPK: em_tile_kernel<COV, XT, DP, CW, MODE_STATS_TOPK><<<grid, block, 0, s>>>(a); break;
-    case MODE_STATS_LSE: em_tile_kernel<COV, XT, DP, CW, MODE_STATS_LSE><<<grid, block, 0, s>>>(a); break;
-    case MODE_PROBA_LSE: em_tile_kernel<COV, XT, DP, CW, MODE_PROBA_LSE><<<grid, block, 0, s>>>(a); break;
+    case MODE_LSE: em_tile_kernel<COV, XT, DP, CW, MODE_LSE, EX><<<grid, block, 0, s>>>(a); break;
+    case MODE_LSE_IDX: em_tile_kernel<COV, XT, DP, CW, MODE_LSE_IDX, EX><<<grid, block, 0, s>>>(a); break;
+    case MODE_IDX: em_tile_kernel<COV, XT, DP, CW, MODE_IDX, EX><<<grid, block, 0, s>>>(a); break;
+    case MODE_STATS: em_tile_kernel<COV, XT, DP, CW, MODE_STATS, EX><<<grid, block, 0, s>>>(a); break;
+    case MODE_PROBA: em_tile_kernel<COV, XT, DP, CW, MODE_PROBA, EX><<<grid, block, 0, s>>>(a); break;
+    case MODE_STATS_TOPK: em_tile_kernel<COV, XT, DP, CW, MODE_STATS_TOPK, EX><<<grid, block, 0, s>>>(a); break;
+    case MODE_STATS_LSE: em_tile_kernel<COV, XT, DP, CW, MODE_STATS_LSE, EX><<<grid, block, 0, s>>>(a); break;
+    case MODE_PROBA_LSE: em_tile_kernel<COV, XT, DP, CW, MODE_PROBA_LSE, EX><<<grid, block, 0, s>>>(a); break;
     default: return -1;
   }
   return 0;
@@ -1253,7 +1300,9 @@ int launch_tile(int cov, int bf, int dp, int mode, const TileArgs& a, dim3 grid,
     case TIED:
       return bf ? -1 : launch_tile_dp<TIED, float>(dp, mode, a, grid, nw, s);
     case FULL:
-      return (bf || dp != 16) ? -1 : launch_tile_t<FULL, float, 16>(mode, a, grid, nw, s);
+      if (bf || dp != 16) return -1;
+      return a.D == 16 ? launch_tile_t<FULL, float, 16, true>(mode, a, grid, nw, s)
+                       : launch_tile_t<FULL, float, 16>(mode, a, grid, nw, s);
     default:
       return -1;
   }

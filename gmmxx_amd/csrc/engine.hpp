@@ -8,7 +8,7 @@ namespace gx {
 
 struct TileArgs {
   const void* x;               // [B][N][D], fp32 or bf16
-  int vec_ok;                  // x rows are 16-byte aligned and D == DP
+  int vec_ok;                  // bf16: x rows are 16-byte aligned and D == DP
   int64_t N;
   int D, K, B;
   int ktiles;                  // component tiles per batch
@@ -28,6 +28,7 @@ struct TileArgs {
   float* part_stats;           // [slices][B][K][JP]                    (STATS)
   float* proba;                // [B][N][K]                             (PROBA)
   float* scores;               // [B][N] natural-log row log-normalisers (PROBA_LSE, or null)
+  int64_t* labels;             // [B][N] first argmax (IDX with ktiles == 1, or null: partials)
   int nslices;                 // row slices of the fused kernel
   double* ll_part;             // [B][nslices] partial log-likelihood   (fused)
   int raw_logits;              // PROBA: write the log2-domain logits instead of responsibilities

@@ -838,6 +838,13 @@ __global__ void combine_kernel(CombineArgs a) {
     for (int t = 0; t < a.ktiles; ++t) {
       const size_t o = ((size_t)t * a.B + b) * a.N + n;
       // Argmax partials exist only when the tile pass tracked them (labels requested).
+      if (a.max_only) {         // (the pass formed no sums)
+        const float m2 = a.part_ms[2 * o];
+        const int i2 = a.part_idx[o];
+        if (m2 > m || (m2 == m && i2 < idx)) idx = i2;
+        m = fmaxf(m, m2);
+        continue;
+      }
       lse_merge(m, s, idx, a.part_ms[2 * o], a.part_ms[2 * o + 1], (a.labels || a.idx32) ? a.part_idx[o] : 0);
     }
     const float lse2 = a.max_only ? m : m + __log2f(s);

@@ -50,12 +50,6 @@ __device__ __forceinline__ float group_max(float v) {
   return v;
 }
 
-// 16 bytes at any element address (a bf16 row of odd D starts on a 2-byte boundary).
-struct __attribute__((packed, aligned(2))) Bytes16 { uint32_t w[4]; };
-__device__ __forceinline__ uint4 ld16_any(const __bf16* p) {
-  const Bytes16 v = *reinterpret_cast<const Bytes16*>(p);
-  return make_uint4(v.w[0], v.w[1], v.w[2], v.w[3]);
-}
 // v shifted down by s elements of 16 bits (0 <= s; 8 or more: all zero).
 __device__ __forceinline__ uint4 shift_elems(uint4 v, int s) {
   if (s & 4) { v.x = v.z; v.y = v.w; v.z = 0u; v.w = 0u; }
