@@ -93,6 +93,7 @@ def _declare(lib):
         "gmmxx_hip_finalize_stats": (ctypes.c_int, [P, vp, vp, vp, vp, f64, f64, vp, vp, vp, vp, i64, vp]),
         "gmmxx_hip_kmeans_pp_workspace_bytes": (i64, [i64, i64, i64, i64, ctypes.c_int]),
         "gmmxx_hip_kmeans_pp": (ctypes.c_int, [vp, i64, i64, i64, i64, ctypes.c_int, vp, vp, vp, vp, i64, vp]),
+        "gmmxx_hip_lloyd_update": (ctypes.c_int, [i64, i64, i64, vp, vp, vp, vp, vp]),
         "gmmxx_hip_topk_workspace_bytes": (i64, [P, ctypes.c_int]),
         "gmmxx_hip_estep_stats_topk": (ctypes.c_int, [P, vp, vp, vp, vp, f64, f64, ctypes.c_int, vp, vp, vp,
                                                       vp, vp, i64, vp]),
@@ -111,7 +112,8 @@ def exported_symbols() -> Tuple[str, ...]:
             "gmmxx_hip_estep_stats", "gmmxx_hip_score", "gmmxx_hip_predict_proba",
             "gmmxx_hip_predict_proba_score",
             "gmmxx_hip_gram", "gmmxx_hip_finalize_stats", "gmmxx_hip_topk_workspace_bytes",
-            "gmmxx_hip_estep_stats_topk", "gmmxx_hip_kmeans_pp_workspace_bytes", "gmmxx_hip_kmeans_pp")
+            "gmmxx_hip_estep_stats_topk", "gmmxx_hip_kmeans_pp_workspace_bytes", "gmmxx_hip_kmeans_pp",
+            "gmmxx_hip_lloyd_update")
 
 
 def load_library(path: Optional[str] = None):
@@ -479,6 +481,20 @@ def kmeans_pp(sample: torch.Tensor, n_components: int, first_idx: torch.Tensor, 
                                     _ptr(centers), ctypes.c_void_p(base + (-base) % 256), need, _stream(dev)),
            "gmmxx_hip_kmeans_pp")
     return centers
+
+
+def lloyd_update(nk: torch.Tensor, sum_x: torch.Tensor, means: torch.Tensor, shift: torch.Tensor) -> None:
+    """One Lloyd centre update in place on ``means`` (B, K, D) from a hard assignment's
+    counts and sums; ``shift`` (1 float, device) receives the largest move."""
+    require_hip()
+    for t, nm in ((nk, "nk"), (sum_x, "sum_x"), (means, "means"), (shift, "shift")):
+        if not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()):
+            raise ValueError(f"{nm} must be a contiguous float32 GPU tensor")
+    B, K, D = (int(v) for v in means.shape)
+    if tuple(nk.shape) != (B, K) or tuple(sum_x.shape) != (B, K, D):
+        raise ValueError("nk must have shape (B, K) and sum_x (B, K, D) matching means")
+    _check(_lib.gmmxx_hip_lloyd_update(B, D, K, _ptr(nk), _ptr(sum_x), _ptr(means), _ptr(shift),
+                                       _stream(means.device)), "gmmxx_hip_lloyd_update")
 
 
 def finalize_stats(covariance_type: str, nk: torch.Tensor, sum_x: torch.Tensor, sum_q: Optional[torch.Tensor],

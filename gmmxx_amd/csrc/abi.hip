@@ -1018,9 +1018,13 @@ int gmmxx_hip_estep_stats_topk(const gmmxx_problem* p, const void* x, const floa
     u.thr_idx = thri;
     u.hard = 1;
     if (run_tile(pl, MODE_STATS_TOPK, u, s) != 0) return fail(GMMXX_ERR_UNSUPPORTED, "no tile kernel for this shape");
+    LlFold ll{};
+    ll.part = at<double>(ws, pl.o_ll);
+    ll.count = pl.B * pl.cblocks;
+    ll.inv_total = 1.0;
+    ll.out = ll_sum;
     launch_reduce_slices(u.part_stats, pl.slices, (int64_t)pl.B * pl.K * pl.JP, at<float>(ws, pl.o_stats), s,
-                         red_tmp(pl, ws), red_tmp_floats(pl));
-    launch_ll_reduce(at<double>(ws, pl.o_ll), pl.B * pl.cblocks, 1.0, ll_sum, s);
+                         red_tmp(pl, ws), red_tmp_floats(pl), &ll);
   } else {
   if (pl.bf && pl.cov == SPH && pl.DP >= 128) {
     if ((rc = lse_pass(pl, x, ws, nullptr, nullptr, false, s))) return rc;
@@ -1166,6 +1170,15 @@ int gmmxx_hip_gram(const gmmxx_problem* p, const void* x, float* out, void* ws, 
   launch_gram(reinterpret_cast<const float*>(x), pl.B, pl.N, pl.D, pl.gram_slices, pl.gram_rows, part, s);
   launch_reduce_slices(part, pl.gram_slices, (int64_t)pl.B * pl.D * pl.D, out, s);
   return check_hip("gram");
+}
+
+int gmmxx_hip_lloyd_update(int64_t B, int64_t D, int64_t K, const float* nk, const float* sum_x, float* means,
+                           float* shift, void* stream) {
+  if (B < 1 || D < 1 || K < 1 || B > 65535 || K > 65536 || D > (1 << 20))
+    return fail(GMMXX_ERR_INVALID_ARGUMENT, "B, D and K out of range");
+  if (!nk || !sum_x || !means || !shift) return fail(GMMXX_ERR_INVALID_ARGUMENT, "NULL buffer");
+  launch_lloyd_update(nk, sum_x, means, B * K, (int)D, shift, (hipStream_t)stream);
+  return check_hip("Lloyd update");
 }
 
 int64_t gmmxx_hip_kmeans_pp_workspace_bytes(int64_t B, int64_t S, int64_t D, int64_t K, int trials) {

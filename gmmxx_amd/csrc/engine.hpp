@@ -197,5 +197,8 @@ struct KppArgs {
 int64_t kpp_workspace_bytes(int B, int S, int K, int T);
 void kpp_bind_workspace(KppArgs& a, void* ws);
 void launch_kpp(const KppArgs& a, hipStream_t s);
+// Lloyd update of M centres in place; *shift: the largest Euclidean move.
+void launch_lloyd_update(const float* nk, const float* sum_x, float* means, int64_t M, int D, float* shift,
+                         hipStream_t s);
 
 }  // namespace gx

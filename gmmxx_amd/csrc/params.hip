@@ -1166,26 +1166,28 @@ __global__ void finalize_full_kernel(FinalizeArgs a) {
 }
 
 // Unpacks the statistics rows into (N_k, Σ r x, Σ r q(x)) for callers and tests.
-__global__ void unpack_stats_kernel(UnpackArgs a) {
-  const int b = blockIdx.y;
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+// One wave per component, lanes over the features.
+__global__ __launch_bounds__(256) void unpack_stats_kernel(UnpackArgs a) {
+  const int b = blockIdx.y, lane = threadIdx.x & 63;
+  const int k = blockIdx.x * 4 + threadIdx.x / 64;
   if (k >= a.K) return;
   const size_t bk = (size_t)b * a.K + k;
   const float* sk = a.stats + bk * a.JP;
   const int D = a.D, DP = a.DP;
-  a.nk[bk] = sk[a.nk_col];
-  for (int d = 0; d < D; ++d) a.sum_x[bk * D + d] = sk[d];
+  if (lane == 0) a.nk[bk] = sk[a.nk_col];
+  for (int d = lane; d < D; d += 64) a.sum_x[bk * D + d] = sk[d];
   if (!a.sum_q) return;
   if (a.cov == SPH) {
     float sq = 0.f;
     for (int i = 0; i < a.sq_n; ++i) sq += sk[a.sq_col + i];
-    a.sum_q[bk] = sq;
+    if (lane == 0) a.sum_q[bk] = sq;
   } else if (a.cov == DIAG) {
-    for (int d = 0; d < D; ++d) a.sum_q[bk * D + d] = sk[DP + d];
+    for (int d = lane; d < D; d += 64) a.sum_q[bk * D + d] = sk[DP + d];
   } else if (a.cov == FULL) {
-    for (int d = 0; d < D; ++d)
-      for (int e = 0; e < D; ++e)
-        a.sum_q[(bk * D + d) * D + e] = sk[DP + full_sxx(DP, d < e ? d : e, d < e ? e : d)];
+    for (int t = lane; t < D * D; t += 64) {
+      const int d = t / D, e = t % D;
+      a.sum_q[bk * D * D + t] = sk[DP + full_sxx(DP, d < e ? d : e, d < e ? e : d)];
+    }
   }
 }
 
@@ -1407,7 +1409,7 @@ void launch_finalize(const FinalizeArgs& a, hipStream_t s) {
 }
 
 void launch_unpack(const UnpackArgs& a, int B, hipStream_t s) {
-  unpack_stats_kernel<<<dim3((a.K + 255) / 256, B), 256, 0, s>>>(a);
+  unpack_stats_kernel<<<dim3((a.K + 3) / 4, B), 256, 0, s>>>(a);
 }
 
 void launch_pack(const PackArgs& a, int B, hipStream_t s) {

@@ -116,14 +116,13 @@ def lloyd(x: torch.Tensor, covariance_type: str, centers: torch.Tensor, max_iter
     the statistics being those of the last assignment."""
     k = int(centers.shape[1])
     stats = stats or _HardStats(x, covariance_type, k)
-    means = centers.to(torch.float32).contiguous()
+    means = centers.to(torch.float32).contiguous().clone()
+    shift = torch.empty((1,), dtype=torch.float32, device=means.device)
     nk = sx = sq = None
     n_iter = 0
     for _ in range(max(1, int(max_iters))):
         nk, sx, sq = stats(means)
-        new = torch.where((nk > 0).unsqueeze(-1), sx / nk.clamp_min(1.0).unsqueeze(-1), means).contiguous()
-        shift = (new - means).norm(dim=-1).amax()
-        means = new
+        _hip.lloyd_update(nk, sx, means, shift)
         n_iter += 1
         if tol > 0.0 and float(shift) < tol:
             break

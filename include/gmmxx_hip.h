@@ -270,6 +270,16 @@ int gmmxx_hip_kmeans_pp(const float* sample, int64_t B, int64_t S, int64_t D, in
                         const int64_t* first_idx, const float* draws, float* centers, void* workspace,
                         int64_t workspace_bytes, void* stream);
 
+/* The centre update of one Lloyd iteration, in place on means (B, K, D): a centre
+ * with nk > 0 becomes sum_x / max(nk, 1), an empty cluster keeps its centre, and
+ * shift (device, 1 float) receives the largest Euclidean move of any centre (0 when
+ * none moved; NaN when one became NaN).  nk (B, K) and sum_x (B, K, D) are a hard
+ * assignment's (gmmxx_hip_estep_stats_topk with top_k = 1).  Part of the k-means
+ * initialisation the reference takes from flash-kmeans
+ * (gmmxx/torch_fallback.py:1569-1631). */
+int gmmxx_hip_lloyd_update(int64_t B, int64_t D, int64_t K, const float* nk, const float* sum_x, float* means,
+                           float* shift, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

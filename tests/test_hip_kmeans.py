@@ -165,3 +165,25 @@ def test_without_flash_kmeans_default_init_is_the_reference_random_branch(hip, m
     monkeypatch.setenv("GMMXX_HIP_FLASH_KMEANS", "1")
     est.fit(xd)
     assert est.init_source_ == "kmeans"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,k,d", [(1, 1, 1), (2, 5, 64), (1, 9, 65), (3, 300, 130)])
+def test_lloyd_update(hip, b, k, d):
+    """Centre = mean of its rows, an empty cluster keeps its centre, the largest move:
+    against the formula in float64 (a division and a difference: 1e-6 relative)."""
+    g = torch.Generator().manual_seed(91)
+    nk = torch.randint(0, 4, (b, k), generator=g).float()
+    sx = torch.randn((b, k, d), generator=g) * nk.unsqueeze(-1)
+    means = torch.randn((b, k, d), generator=g)
+    exp = torch.where((nk > 0).unsqueeze(-1), sx.double() / nk.clamp_min(1.0).double().unsqueeze(-1), means.double())
+    m_d, shift = means.cuda(), torch.full((1,), 7.0, device="cuda")
+    for _ in range(2):      # the second update moves nothing
+        move = float((exp - m_d.double().cpu()).norm(dim=-1).amax())
+        hip.lloyd_update(nk.cuda(), sx.cuda(), m_d, shift)
+        torch.testing.assert_close(m_d.cpu().double(), exp, rtol=1e-6, atol=1e-7)
+        assert float(shift) == pytest.approx(move, rel=1e-5, abs=1e-5)
+    means[0, 0, 0] = float("nan")
+    nk[0, 0] = 1.0
+    hip.lloyd_update(nk.cuda(), sx.cuda(), means.cuda(), shift)
+    assert bool(torch.isnan(shift).all())
