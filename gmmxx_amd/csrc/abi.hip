@@ -67,6 +67,7 @@ struct Plan {
   // full covariance at D > 16 (whitening E-step, weighted-Gram statistics)
   bool fw = false;
   int pdt = 0;   // param_dtype
+  bool fw_tile = false;      // statistics by 16-component workgroups (em_full_stats.hip)
   int fw_eblk = 0, fw_slices = 0;
   int64_t fw_rows = 0;
   size_t o_lpack = 0, o_lpaug = 0, o_l2w = 0, o_linv = 0;
@@ -243,14 +244,17 @@ int plan_problem(const gmmxx_problem* p, Plan* pl) {
   q.gram_slices = (int)((q.N + q.gram_rows - 1) / q.gram_rows);
   q.chol_m = (q.cov == TIED) ? q.B : (q.cov == FULL ? q.B * q.K : 0);
   if (q.fw) {
-    // E-step: one wave per 32-row block.  Statistics: workgroups of four waves
-    // (four components; at D = 128 two components of two waves) over row slices,
-    // as many as one round of resident waves: 8, 4 and 2 waves per SIMD at
+    // E-step: one wave per 32-row block.  Statistics: eight-wave workgroups of 16
+    // components over row slices, one per CU (em_full_stats.hip), or, for few
+    // components, workgroups of four waves (four components; at D = 128 two
+    // components of two waves), as many as one round of resident waves: 8, 4 and 2 waves per SIMD at
     // DP = 32, 64 and 128 (the kernels' register counts), so 2048, 1024 and 512
     // workgroups (at D = 64, 2048 measured 5 % slower per EM iteration).
     q.fw_eblk = fw_eblocks(q.N);
-    const int64_t groups = (int64_t)(q.DP == 128 ? (q.K + 1) / 2 : (q.K + 3) / 4) * q.B;
-    const int64_t target = q.DP == 32 ? 2048 : (q.DP == 64 ? 1024 : 512);
+    q.fw_tile = fw_stats_tile_pays(q.D, q.DP, q.K);
+    const int64_t groups =
+        (q.fw_tile ? fw_stats_tile_groups(q.D, q.K) : (q.DP == 128 ? (q.K + 1) / 2 : (q.K + 3) / 4)) * (int64_t)q.B;
+    const int64_t target = q.fw_tile ? 256 : (q.DP == 32 ? 2048 : (q.DP == 64 ? 1024 : 512));
     int64_t fs = std::max<int64_t>(1, (target + groups - 1) / groups);
     fs = std::min(fs, std::max<int64_t>(1, row_blocks / kMinBlocksPerSlice));
     q.fw_rows = ((q.N + fs - 1) / fs + kBN - 1) / kBN * kBN;
@@ -469,6 +473,7 @@ FwArgs fw_args(const Plan& pl, const void* x, void* ws) {
   a.part_stats = at<float>(ws, pl.o_pstats);
   a.JP = pl.JP;
   a.nk_col = pl.nk_col;
+  a.nk_dp = pl.DP;
   a.rows_per_slice = pl.fw_rows;
   return a;
 }
@@ -501,7 +506,8 @@ int run_w16(const Plan& pl, const void* x, const float* means, const float* covs
 }
 
 int run_fw(const Plan& pl, int phase, const FwArgs& a, hipStream_t s) {
-  if (launch_fw(pl.DP, phase, a, pl.fw_slices, s) != 0) return fail(GMMXX_ERR_UNSUPPORTED, "no full-covariance kernel for this D");
+  if ((phase == 1 && pl.fw_tile ? launch_fw_stats_tile(a, pl.fw_slices, s) : launch_fw(pl.DP, phase, a, pl.fw_slices, s)) != 0)
+    return fail(GMMXX_ERR_UNSUPPORTED, "no full-covariance kernel for this D");
   return check_hip(phase == 0 ? "full-covariance E-step" : "full-covariance statistics");
 }
 // Where an EM iteration's tied -½ tr(P XᵀX) terms go: after the log-likelihood

@@ -131,6 +131,7 @@ struct FwArgs {
   double* ll_part;             // [B][fw_eblocks(N)] natural-log partial sums, or null
   float* part_stats;           // [slices][B][K][JP]
   int JP, nk_col;
+  int nk_dp;                   // padded D of the statistics rows (32, 64, 128)
   int64_t rows_per_slice;      // statistics kernel: rows per slice
   // Hard assignment (approximate top-k EM with k = 1): the E-step writes each
   // row's first argmax to hard_idx and its maximum as the log-normaliser; the
@@ -149,6 +150,11 @@ void launch_fw_pack(const FwPackArgs& a, hipStream_t s);
 // phase 0: the E-step over fw_eblocks(N) x B workgroups; 1: the statistics over
 // slices x ceil(K / 4) x B.  Returns -1 for an unsupported dp.
 int launch_fw(int dp, int phase, const FwArgs& a, int slices, hipStream_t s);
+// The statistics by 16-component workgroups (em_full_stats.hip) over slices x
+// fw_stats_tile_groups(D, K) x B; 16 < D <= 128.
+int fw_stats_tile_groups(int D, int K);
+bool fw_stats_tile_pays(int D, int DP, int K);
+int launch_fw_stats_tile(const FwArgs& a, int slices, hipStream_t s);
 // proba[b][n][k] = 2^(l2[b][k][n] - lse2[b][n]), or (raw) the log2 logits l2 themselves, transposed.
 void launch_fw_proba(const float* l2, const float* lse2, float* proba, int B, int64_t N, int K, hipStream_t s,
                      bool raw = false);
