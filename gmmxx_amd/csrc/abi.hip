@@ -159,7 +159,9 @@ int plan_problem(const gmmxx_problem* p, Plan* pl) {
   const int64_t row_blocks = (q.N + kBN - 1) / kBN;
   const int64_t target_blocks = (kTargetWaves + q.nw - 1) / q.nw;
   int64_t slices = std::max<int64_t>(1, (target_blocks + (int64_t)q.ktiles * q.B - 1) / ((int64_t)q.ktiles * q.B));
-  slices = std::min(slices, std::max<int64_t>(1, row_blocks / kMinBlocksPerSlice));
+  // (problems that leave most CUs idle: one block per slice, the shortest chain)
+  const int64_t min_blocks = row_blocks * q.ktiles * q.B <= 256 ? 1 : kMinBlocksPerSlice;
+  slices = std::min(slices, std::max<int64_t>(1, row_blocks / min_blocks));
   q.rows_per_slice = ((q.N + slices - 1) / slices + kBN - 1) / kBN * kBN;
   q.slices = (int)((q.N + q.rows_per_slice - 1) / q.rows_per_slice);
   q.cblocks = combine_blocks(q.N);
@@ -854,12 +856,28 @@ int gmmxx_hip_em_phase(const gmmxx_problem* p, int phase, const void* x, float* 
 int gmmxx_hip_em_step(const gmmxx_problem* p, const void* x, float* means, float* covs, float* weights,
                       const float* gram, double reg_covar, double min_weight, float* lower_bound,
                       void* ws, int64_t ws_bytes, void* stream) {
-  for (int ph = GMMXX_PHASE_PREPARE; ph <= GMMXX_PHASE_FINALIZE; ++ph) {
+  int last = GMMXX_PHASE_FINALIZE;
+  // A single pass with small statistics: the reduction and the finalize share a launch.
+  Plan pl;
+  int prc = plan_problem(p, &pl);
+  if (prc) return prc;
+  FinalizeArgs f{};
+  const bool fuse = ll_in_pass(pl) && !(pl.coop && pl.cG > 1) && !pl.xch && ws && (f = finalize_args(
+      pl, ws, gram, reg_covar, min_weight, pl.N, means, covs, weights, nullptr),
+      reduce_finalize_fits(f, stat_slices(pl), red_tmp_floats(pl)));
+  if (fuse) last = GMMXX_PHASE_STATS_TILE;
+  for (int ph = GMMXX_PHASE_PREPARE; ph <= last; ++ph) {
     const int rc = gmmxx_hip_em_phase(p, ph, x, means, covs, weights, gram, reg_covar, min_weight,
                                       lower_bound, ws, ws_bytes, stream);
     if (rc) return rc;
   }
-  return GMMXX_OK;
+  if (!fuse) return GMMXX_OK;
+  int parts = ll_parts(pl);
+  if (tied_shift(pl, ws)) parts += pl.B * pl.D;   // -½ tr(P XᵀX) rows, from the prepare phase
+  launch_reduce_finalize(f, at<float>(ws, pl.o_pstats), stat_slices(pl), red_tmp(pl, ws), red_tmp_floats(pl),
+                         ll_fold(pl, ws, parts, 1.0 / ((double)pl.B * (double)pl.N), lower_bound),
+                         (hipStream_t)stream);
+  return check_hip("reduction and finalize");
 }
 
 int gmmxx_hip_em_step_noalloc(const gmmxx_problem* p, const void* x, float* means, float* covs, float* weights,

@@ -1058,11 +1058,11 @@ __device__ float finalize_total(const FinalizeArgs& a, int b, float* scratch) {
 // Component k of batch b, one wave (lanes over the features): w_new =
 // max(N_k / N, min_weight) / total (torch_fallback.py:2303-2305); means and
 // spherical/diag variances with the active mask (:2293-2302, :2654-2666).
-__device__ void finalize_comp(const FinalizeArgs& a, int b, int k, float total) {
+// sk: the component's statistics row (global memory or LDS).
+__device__ __forceinline__ void finalize_comp(const FinalizeArgs& a, int b, int k, const float* sk, float total) {
   const int lane = threadIdx.x & 63;
   const int D = a.D;
   const size_t bk = (size_t)b * a.K + k;
-  const float* sk = a.stats + bk * a.JP;
   const float nk = sk[a.nk_col];
   const bool active = nk > a.min_weight;
   const float nk_safe = clamp_lo(nk, a.min_weight);
@@ -1104,7 +1104,7 @@ __global__ __launch_bounds__(64 * kFinWaves) void finalize_kernel(FinalizeArgs a
   const int b = blockIdx.y;
   const float total = finalize_total(a, b, scratch);
   const int k = blockIdx.x * kFinWaves + threadIdx.x / 64;
-  if (k < a.K) finalize_comp(a, b, k, total);
+  if (k < a.K) finalize_comp(a, b, k, a.stats + ((size_t)b * a.K + k) * a.JP, total);
 }
 
 // Tied: Σ = sym((XᵀX − Σ_k n_k μ_k μ_kᵀ) / N) + reg·I   (torch_fallback.py:3159-3162)
@@ -1144,12 +1144,9 @@ __global__ __launch_bounds__(64 * kTiedWaves) void finalize_tied_kernel(Finalize
 }
 
 // Full: Σ_k = sym((Σ r xxᵀ − n_k μμᵀ) / max(n_k, floor)) + reg·I, kept if inactive (:3150-3158)
-__global__ void finalize_full_kernel(FinalizeArgs a) {
-  const int b = blockIdx.y, k = blockIdx.x;
-  const int K = a.K, D = a.D, JP = a.JP, DP = a.DP;
-  if (a.skip && *a.skip != 0u) return;
+__device__ __forceinline__ void finalize_full_comp(const FinalizeArgs& a, int b, int k, const float* sk) {
+  const int K = a.K, D = a.D, DP = a.DP;
   const size_t bk = (size_t)b * K + k;
-  const float* sk = a.stats + bk * JP;
   const float nk = sk[a.nk_col];
   const bool active = nk > a.min_weight;
   const float nk_safe = clamp_lo(nk, a.min_weight);
@@ -1162,6 +1159,82 @@ __global__ void finalize_full_kernel(FinalizeArgs a) {
     const float aed = (sxx - nk * (mu[e] * mu[d])) / nk_safe;
     const float v = 0.5f * (ade + aed) + (d == e ? a.reg_covar : 0.f);
     if (active) C[t] = round_param(v, a.param_round);  // inactive components keep their previous covariance
+  }
+}
+__global__ void finalize_full_kernel(FinalizeArgs a) {
+  if (a.skip && *a.skip != 0u) return;
+  finalize_full_comp(a, blockIdx.y, blockIdx.x, a.stats + ((size_t)blockIdx.y * a.K + blockIdx.x) * a.JP);
+}
+
+// The last slice reduction and the finalize in one launch, one workgroup per
+// component: sums its statistics row over the `slices` partials (wave g the slices
+// g, g + 16, ..., then the wave sums in wave order: reduce_slices_kernel's order and
+// bits), forms every component's N_k the same way for the weights' total, and
+// updates its own parameters (full: the covariance too).  blockIdx.x == K: the
+// log-likelihood.  A dependent launch costs about 5 µs here whatever it does, so
+// for small statistics the launch it saves (two for full) is worth every workgroup
+// re-reading all N_k: K · slices values, at most kFusedFinLoads (at 6656, spherical
+// N = 10000, D = 32, K = 64, the iteration lost 1.7 of 25 µs), and at most kFusedFinK
+// components over all problems (one workgroup per CU; at 512, full 16 x 262144,
+// D = 16, it gained nothing).  Iteration at
+// N = 100000, D = 32, K = 64: 40.0 -> 36.3 µs; full N = 1500, D = 4, K = 3: 42.6 -> 39.9.
+constexpr int kFusedFinLoads = 4096;
+constexpr int kFusedFinJP = 512, kFusedFinK = 256;
+__global__ __launch_bounds__(64 * kRedWaves) void reduce_finalize_kernel(FinalizeArgs a, const float* part, int slices,
+                                                                         float* stats, LlFold ll) {
+  __shared__ float red[kRedWaves][kFusedFinJP];
+  __shared__ float row[kFusedFinJP];
+  __shared__ float nkp[kFusedFinK * kRedWaves];
+  __shared__ float scratch[32];
+  const int b = blockIdx.y, k = blockIdx.x, tid = threadIdx.x, lane = tid & 63, g = tid >> 6;
+  const int K = a.K, JP = a.JP;
+  if (k == K) {
+    __shared__ double dscratch[32];
+    if (b != 0) return;
+    double t = 0.0;
+    for (int i = tid; i < ll.count; i += blockDim.x) t += ll.part[i];
+    t = block_sum(t, dscratch);
+    if (tid == 0) ll.out[0] = (float)(t * ll.inv_total);
+    return;
+  }
+  const int64_t M = (int64_t)a.B * K * JP;
+  const float* prow = part + ((size_t)b * K + k) * JP;
+  for (int c = lane; c < JP; c += 64) {
+    float s = 0.f;
+#pragma unroll 4
+    for (int t = g; t < slices; t += kRedWaves) s += prow[(size_t)t * M + c];
+    red[g][c] = s;
+  }
+  // Σ_k max(N_k / N, min_weight), the terms as finalize_total adds them: every
+  // (component, wave) partial sum on its own thread first, so no thread walks all
+  // slices.
+  const float* pn = part + (size_t)b * K * JP + a.nk_col;
+  for (int e = tid; e < K * kRedWaves; e += blockDim.x) {
+    const int k2 = e / kRedWaves, w = e % kRedWaves;
+    float s = 0.f;
+#pragma unroll 4
+    for (int t = w; t < slices; t += kRedWaves) s += pn[(size_t)t * M + (size_t)k2 * JP];
+    nkp[e] = s;
+  }
+  __syncthreads();
+  float wsum = 0.f;
+  for (int k2 = tid; k2 < K; k2 += blockDim.x) {
+    float nk = nkp[k2 * kRedWaves];
+    for (int w = 1; w < kRedWaves; ++w) nk += nkp[k2 * kRedWaves + w];
+    wsum += clamp_lo(nk / (float)a.N, a.min_weight);
+  }
+  const float total = block_sum(wsum, scratch);   // (its barriers also cover red)
+  for (int c = tid; c < JP; c += blockDim.x) {
+    float tot = red[0][c];
+    for (int w = 1; w < kRedWaves; ++w) tot += red[w][c];
+    row[c] = tot;
+    if (stats) stats[((size_t)b * K + k) * JP + c] = tot;
+  }
+  __syncthreads();
+  if (g == 0) finalize_comp(a, b, k, row, total);
+  if (a.cov == FULL) {
+    __syncthreads();                              // the new mean, written by wave 0
+    finalize_full_comp(a, b, k, row);
   }
 }
 
@@ -1360,26 +1433,56 @@ void launch_ll_reduce(const double* ll_part, int count, double inv_total, float*
   ll_reduce_kernel<<<1, 1024, 0, s>>>(ll_part, count, inv_total, out);
 }
 
-void launch_reduce_slices(const float* part, int slices, int64_t M, float* out, hipStream_t s, float* tmp,
-                          int64_t tmp_floats, const LlFold* ll) {
-  // Many slices over few outputs: first sum groups of slices in parallel into
-  // tmp (fixed grouping, so the result stays deterministic), then the groups.
+// Groups of slices summed in parallel before the last reduction (1: none): many
+// slices over few outputs, a fixed grouping, so the result stays deterministic.
+static int reduce_groups(int slices, int64_t M, int64_t tmp_floats) {
   const int64_t blocks = (M + 63) / 64;
   int groups = 1;
   while (groups < 64 && blocks * groups < 512 && slices / (2 * groups) >= 4 * kRedWaves &&
          (int64_t)(2 * groups) * M <= tmp_floats)
     groups *= 2;
-  const LlFold none{};
-  const LlFold lf = ll ? *ll : none;
-  const unsigned last = (unsigned)blocks + (ll ? 1u : 0u);
-  if (groups == 1 || !tmp) {
-    reduce_slices_kernel<<<last, 64 * kRedWaves, 0, s>>>(part, slices, M, out, slices, lf);
-    return;
-  }
+  return groups;
+}
+
+// The first stage: `groups` sums of consecutive slices into tmp; returns how many.
+static int reduce_first(const float* part, int slices, int64_t M, int groups, float* tmp, hipStream_t s) {
   const int per = (slices + groups - 1) / groups;
   groups = (slices + per - 1) / per;  // every group non-empty
-  reduce_slices_kernel<<<dim3((unsigned)blocks, groups), 64 * kRedWaves, 0, s>>>(part, slices, M, tmp, per, none);
-  reduce_slices_kernel<<<last, 64 * kRedWaves, 0, s>>>(tmp, groups, M, out, groups, lf);
+  reduce_slices_kernel<<<dim3((unsigned)((M + 63) / 64), groups), 64 * kRedWaves, 0, s>>>(part, slices, M, tmp, per,
+                                                                                          LlFold{});
+  return groups;
+}
+
+void launch_reduce_slices(const float* part, int slices, int64_t M, float* out, hipStream_t s, float* tmp,
+                          int64_t tmp_floats, const LlFold* ll) {
+  const int groups = tmp ? reduce_groups(slices, M, tmp_floats) : 1;
+  const LlFold lf = ll ? *ll : LlFold{};
+  const unsigned last = (unsigned)((M + 63) / 64) + (ll ? 1u : 0u);
+  if (groups > 1) {
+    slices = reduce_first(part, slices, M, groups, tmp, s);
+    part = tmp;
+  }
+  reduce_slices_kernel<<<last, 64 * kRedWaves, 0, s>>>(part, slices, M, out, slices, lf);
+}
+
+bool reduce_finalize_fits(const FinalizeArgs& a, int slices, int64_t tmp_floats) {
+  const int64_t M = (int64_t)a.B * a.K * a.JP;
+  const int groups = reduce_groups(slices, M, tmp_floats);
+  return !a.skip && a.JP <= kFusedFinJP && (int64_t)a.B * a.K <= kFusedFinK && (int64_t)a.K * (groups > 1 ? groups : slices) <= kFusedFinLoads;
+}
+
+void launch_reduce_finalize(const FinalizeArgs& a, const float* part, int slices, float* tmp, int64_t tmp_floats,
+                            const LlFold& ll, hipStream_t s) {
+  const int64_t M = (int64_t)a.B * a.K * a.JP;
+  const int groups = reduce_groups(slices, M, tmp_floats);
+  if (groups > 1) {
+    slices = reduce_first(part, slices, M, groups, tmp, s);
+    part = tmp;
+  }
+  // (tied: its covariance update reads the statistics rows)
+  reduce_finalize_kernel<<<dim3(a.K + 1, a.B), 64 * kRedWaves, 0, s>>>(a, part, slices,
+                                                                      a.cov == TIED ? const_cast<float*>(a.stats) : nullptr, ll);
+  if (a.cov == TIED) finalize_tied_kernel<<<dim3(a.D, a.B, (a.D + 63) / 64), 64 * kTiedWaves, 0, s>>>(a);
 }
 
 __global__ void take_status_kernel(unsigned* sticky, uint32_t* out) {

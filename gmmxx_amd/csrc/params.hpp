@@ -113,6 +113,11 @@ struct LlFold {
 void launch_reduce_slices(const float* part, int slices, int64_t M, float* out, hipStream_t s,
                           float* tmp = nullptr, int64_t tmp_floats = 0, const LlFold* ll = nullptr);
 void launch_finalize(const FinalizeArgs& a, hipStream_t s);
+// Slice reduction, log-likelihood (its status words unused) and finalize with the
+// last reduction and the finalize in one launch, for statistics small enough.
+bool reduce_finalize_fits(const FinalizeArgs& a, int slices, int64_t tmp_floats);
+void launch_reduce_finalize(const FinalizeArgs& a, const float* part, int slices, float* tmp, int64_t tmp_floats,
+                            const LlFold& ll, hipStream_t s);
 void launch_unpack(const UnpackArgs& a, int B, hipStream_t s);
 void launch_pack(const PackArgs& a, int B, hipStream_t s);
 void launch_gram(const float* x, int B, int64_t N, int D, int slices, int64_t rows_per_slice, float* part,
