@@ -82,6 +82,8 @@ def _declare(lib):
         "gmmxx_hip_device_info": (ctypes.c_int, [ctypes.c_int, ctypes.POINTER(DevInfo)]),
         "gmmxx_hip_take_status": (ctypes.c_int, [P, vp, i64, vp, vp]),
         "gmmxx_hip_workspace_bytes": (i64, [P]),
+        "gmmxx_hip_exchanges": (ctypes.c_int, [P]),
+        "gmmxx_hip_workspace_init": (ctypes.c_int, [P, vp, i64, vp]),
         "gmmxx_hip_em_step": (ctypes.c_int, [P, vp, vp, vp, vp, vp, f64, f64, vp, vp, i64, vp]),
         "gmmxx_hip_em_step_noalloc": (ctypes.c_int, [P, vp, vp, vp, vp, vp, f64, f64, vp, vp]),
         "gmmxx_hip_em_phase": (ctypes.c_int, [P, ctypes.c_int, vp, vp, vp, vp, vp, f64, f64, vp, vp, i64, vp]),
@@ -113,7 +115,7 @@ def exported_symbols() -> Tuple[str, ...]:
             "gmmxx_hip_predict_proba_score",
             "gmmxx_hip_gram", "gmmxx_hip_finalize_stats", "gmmxx_hip_topk_workspace_bytes",
             "gmmxx_hip_estep_stats_topk", "gmmxx_hip_kmeans_pp_workspace_bytes", "gmmxx_hip_kmeans_pp",
-            "gmmxx_hip_lloyd_update")
+            "gmmxx_hip_lloyd_update", "gmmxx_hip_exchanges", "gmmxx_hip_workspace_init")
 
 
 def load_library(path: Optional[str] = None):
@@ -226,13 +228,20 @@ class Workspace:
         if nbytes < 0:
             raise HipRuntimeError("problem not supported by the HIP engine: "
                                   + lib.gmmxx_hip_last_error().decode(errors="replace"))
-        # Zeroed once: the asynchronous status word (gmmxx_hip_take_status) starts clear.
-        self._buf = torch.zeros(nbytes + 256, dtype=torch.uint8, device=device)
+        # Not zeroed: every byte but the asynchronous status words is written before it is
+        # read, and those exist only for problems whose workgroups exchange partials
+        # (filling the whole buffer cost 14 us per predict_proba call at B = 16,
+        # N = 262144, and a launch for the smallest).
+        self._buf = torch.empty(nbytes + 256, dtype=torch.uint8, device=device)
         base = self._buf.data_ptr()
         self.ptr = ctypes.c_void_p(base + (-base) % 256)
         self.nbytes = nbytes
         self.prob = prob
-        self.device = torch.device(device)
+        self.device = self._buf.device
+        self.exchanges = bool(lib.gmmxx_hip_exchanges(ctypes.byref(prob)))
+        if self.exchanges:
+            _check(lib.gmmxx_hip_workspace_init(ctypes.byref(prob), self.ptr, nbytes, _stream(self.device)),
+                   "gmmxx_hip_workspace_init")
 
 
 def take_status(ws: Workspace) -> torch.Tensor:
@@ -242,7 +251,7 @@ def take_status(ws: Workspace) -> torch.Tensor:
     waiting for a partner; its iteration kept the parameters and wrote a NaN
     lower bound).  Clears it;
     stream-ordered, no synchronisation."""
-    out = torch.zeros((1,), dtype=torch.int32, device=ws.device)
+    out = torch.empty((1,), dtype=torch.int32, device=ws.device)
     _check(_lib.gmmxx_hip_take_status(ctypes.byref(ws.prob), ws.ptr, ws.nbytes, _ptr(out), _stream(ws.device)),
            "gmmxx_hip_take_status")
     return out

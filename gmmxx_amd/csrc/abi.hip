@@ -50,6 +50,7 @@ struct Plan {
   bool coop = false;         // EM iteration as one cooperative pass (spherical bf16; em_coop.hip)
   bool single = false;       // EM iteration as one tile pass (fp32 x, all K in one workgroup; MODE_STATS_LSE)
   bool xch = false;          // EM iteration as one tile pass whose 2..4 component tiles exchange row partials
+  bool may_exchange = false; // coop or xch groups, whatever GMMXX_HIP_NO_COOP / _NO_XCH say
   int xslices = 0;           // xch: row slices per batch (grid xslices·ktiles x B, all resident)
   int64_t xrows = 0;         // xch: rows per slice
   int cDP = 0, cnw = 0;      // coop: padded row width, waves per workgroup
@@ -230,6 +231,9 @@ int plan_problem(const gmmxx_problem* p, Plan* pl) {
   const char* no_xch = getenv("GMMXX_HIP_NO_XCH");
   q.xch = !q.bf && (q.cov == SPH || q.cov == TIED || (q.cov == DIAG && q.DP <= 64)) && q.ktiles >= 2 &&
           q.ktiles <= kMaxCoopGroup && q.nw == 8 && !(no_xch && no_xch[0] == '1');
+  q.may_exchange = (sph_bf && !q.fused && q.K > kCoopComps && q.K <= kCoopComps * kMaxCoopGroup) ||
+                   (!q.bf && (q.cov == SPH || q.cov == TIED || (q.cov == DIAG && q.DP <= 64)) && q.ktiles >= 2 &&
+                    q.ktiles <= kMaxCoopGroup && q.nw == 8);
   if (q.xch) {
     int64_t xs = tile_xch_capacity(q.cov, q.DP) / ((int64_t)q.ktiles * q.B);
     xs = std::min(xs, std::max<int64_t>(1, row_blocks / kMinBlocksPerSlice));
@@ -774,8 +778,26 @@ int gmmxx_hip_take_status(const gmmxx_problem* p, void* ws, int64_t ws_bytes, ui
   if (rc) return rc;
   if ((rc = check_ws(pl, ws, ws_bytes))) return rc;
   if (!status_out) return fail(GMMXX_ERR_INVALID_ARGUMENT, "status_out is NULL");
-  launch_take_status(sticky_status(pl, ws), status_out, (hipStream_t)stream);
+  if (pl.may_exchange) launch_take_status(sticky_status(pl, ws), status_out, (hipStream_t)stream);
+  else launch_zero_words(status_out, 1, (hipStream_t)stream);   // (nothing writes the status words)
   return check_hip("take_status");
+}
+
+int gmmxx_hip_exchanges(const gmmxx_problem* p) {
+  Plan pl;
+  const std::string saved = g_last_error;
+  const int rc = plan_problem(p, &pl);
+  g_last_error = saved;
+  return rc == GMMXX_OK && pl.may_exchange ? 1 : 0;
+}
+
+int gmmxx_hip_workspace_init(const gmmxx_problem* p, void* ws, int64_t ws_bytes, void* stream) {
+  Plan pl;
+  int rc = plan_problem(p, &pl);
+  if (rc) return rc;
+  if ((rc = check_ws(pl, ws, ws_bytes))) return rc;
+  if (pl.may_exchange) launch_zero_words(at<unsigned>(ws, pl.o_flags), 2, (hipStream_t)stream);
+  return check_hip("workspace_init");
 }
 
 int gmmxx_hip_em_phase(const gmmxx_problem* p, int phase, const void* x, float* means, float* covs,

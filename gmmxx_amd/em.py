@@ -317,7 +317,7 @@ def fit(x: torch.Tensor, n_components: int, covariance_type: str, *, max_iters: 
         ws = None
         topk_step = _TopkStep(x, covariance_type, k, top_k, param_dtype)
         gram = topk_step.gram() if covariance_type == "tied" else None
-    lb = torch.zeros((max_iters,), dtype=torch.float32, device=x.device)
+    lb = torch.empty((max_iters,), dtype=torch.float32, device=x.device)   # (each iteration writes its own)
     spherical = covariance_type == "spherical"
     sync_each = bool(verbose or tol > 0.0)
     prev = None
@@ -346,7 +346,7 @@ def fit(x: torch.Tensor, n_components: int, covariance_type: str, *, max_iters: 
                 break
             if tol > 0.0:
                 prev = value
-    if ws is not None:
+    if ws is not None and ws.exchanges:
         # A cooperative pass that gave up waiting left its iteration's parameters
         # unchanged and a NaN lower bound; the fit reports it instead of returning.
         _hip.raise_on_status(_hip.take_status(ws), "EM fit")

@@ -122,12 +122,23 @@ int gmmxx_hip_em_step(const gmmxx_problem* p, const void* x, float* means, float
  * exchange: it propagates into the lower bound and parameters as in the
  * reference, and the word stays 0.  Copies the word into *status_out (device
  * memory, 1 uint32) and clears it, stream-ordered.  A newly allocated workspace holds arbitrary
- * bytes: zero it, or call this once and discard the result, before the calls
+ * bytes: gmmxx_hip_workspace_init it (or zero it, or call this once and discard the
+ * result) before the calls
  * whose status is wanted.  No reference counterpart: the reference's kernels
  * report errors synchronously through TORCH_CHECK (gmmxx/_cuda.py:41-54); this
  * is how the asynchronous C ABI reports its one asynchronous failure. */
 int gmmxx_hip_take_status(const gmmxx_problem* p, void* workspace, int64_t workspace_bytes,
                           uint32_t* status_out, void* stream);
+
+/* 1 if passes of this problem may exchange row partials (see
+ * gmmxx_hip_take_status, whose word then means something; otherwise it is 0), 0 if
+ * not or unsupported. */
+int gmmxx_hip_exchanges(const gmmxx_problem* p);
+
+/* Clears the status words of a newly allocated workspace (the only bytes a call reads
+ * before one writes them; nothing to do, and nothing launched, for problems that
+ * never exchange). */
+int gmmxx_hip_workspace_init(const gmmxx_problem* p, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* gmmxx_hip_em_step without a caller workspace: the same kernels run on a
  * static device scratch array of the library (64 MiB per device, held for
