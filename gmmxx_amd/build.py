@@ -19,7 +19,7 @@ ROOT = os.path.dirname(PKG_DIR)
 CSRC = os.path.join(PKG_DIR, "csrc")
 BUILD_DIR = os.path.join(PKG_DIR, "_build")
 LIB_PATH = os.path.join(PKG_DIR, "libgmmxx_hip.so")
-SOURCES = ("em_tile.hip", "em_sph_bf16.hip", "em_fused.hip", "em_coop.hip", "em_one.hip", "em_full_wide.hip", "em_full_stats.hip", "em_full_infer.hip",
+SOURCES = ("em_tile.hip", "em_sph_bf16.hip", "em_fused.hip", "em_coop.hip", "em_one.hip", "em_label.hip", "em_full_wide.hip", "em_full_stats.hip", "em_full_infer.hip",
            "params.hip",
            "kmeans.hip", "abi.hip")
 ARCH = os.environ.get("GMMXX_HIP_ARCH", "gfx950")
@@ -36,7 +36,8 @@ EXTRA_FLAGS = {"em_tile.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"],
                "em_sph_bf16.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"],
                "em_fused.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"],
                "em_coop.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"],
-               "em_one.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"]}
+               "em_one.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"],
+               "em_label.hip": ["-fno-honor-nans", "-mno-amdgpu-ieee"]}
 
 
 def _hipcc() -> str:

@@ -47,6 +47,7 @@ struct Plan {
   int DP = 0, EP = 0, JP = 0, nk_col = 0, sq_col = 0, sq_n = 0, CW = 0, nw = 0, ktiles = 0, slices = 0, cblocks = 0;
   int lnw = 0, lktiles = 0;  // waves / component tiles of the plain log-normaliser pass (MODE_LSE)
   bool fused = false;        // EM iteration as one fused pass (small K; em_fused.hip)
+  bool sb = false;           // spherical bf16 operands of the single passes and the label pass
   bool coop = false;         // EM iteration as one cooperative pass (spherical bf16; em_coop.hip)
   bool single = false;       // EM iteration as one tile pass (fp32 x, all K in one workgroup; MODE_STATS_LSE)
   bool xch = false;          // EM iteration as one tile pass whose 2..4 component tiles exchange row partials
@@ -277,10 +278,12 @@ int plan_problem(const gmmxx_problem* p, Plan* pl) {
   q.o_whi = take(BK * q.EP * (q.bf ? 2 : 4));
   q.o_wlo = take(q.bf ? BK * q.EP * 2 : 0);
   q.o_waug = take(sph_bf ? BK * 32 * 2 : 0);
-  q.o_wmu = take((q.coop || q.fused) ? BK * q.DP * 2 : 0);
-  q.o_wsc = take((q.coop || q.fused) ? BK * 4 : 0);
-  const bool one_group = q.fused || (q.coop && q.cG == 1);   // logits as s·(x·μ - ‖x‖²/2 + C')
-  q.o_waugs = take(one_group ? BK * 16 * 2 : 0);
+  // The bf16 means, their factor and the augmented constants of s·(x·μ - ‖x‖²/2 + C'):
+  // the single passes and the label pass.
+  q.sb = sph_bf && q.K <= kCoopComps * kMaxCoopGroup;
+  q.o_wmu = take(q.sb ? BK * q.DP * 2 : 0);
+  q.o_wsc = take(q.sb ? BK * 4 : 0);
+  q.o_waugs = take(q.sb ? BK * 16 * 2 : 0);
   q.o_cconst = take(BK * 16);
   q.o_covs_used = take(q.cov == SPH ? BK * 4 : (q.cov == DIAG ? BK * q.D * 4 : 0));
   q.o_rowq = take(q.cov == TIED ? BN * 4 : 0);
@@ -381,9 +384,7 @@ int run_fused(const Plan& pl, const TileArgs& t, hipStream_t s) {
   return launch_sph_bf16_fused(pl.DP, pl.K, u, pl.fslices, s);
 }
 // Cooperative single pass: partial statistics per row item and partial log-likelihoods.
-int run_coop(const Plan& pl, const void* x, void* ws, hipStream_t s) {
-  if (pl.D == 128 && pl.cG > 1 && (uintptr_t)x % 16 != 0)
-    return fail(GMMXX_ERR_INVALID_ARGUMENT, "x must be 16-byte aligned for spherical bf16 at D = 128");
+CoopArgs sb_args(const Plan& pl, const void* x, void* ws) {
   CoopArgs c{};
   c.x = x;
   c.vec = pl.D % 8 == 0 && (uintptr_t)x % 16 == 0;
@@ -394,8 +395,14 @@ int run_coop(const Plan& pl, const void* x, void* ws, hipStream_t s) {
   c.B = pl.B;
   c.w_mu = at<void>(ws, pl.o_wmu);
   c.w_scale = at<float>(ws, pl.o_wsc);
-  c.w_aug = at<void>(ws, pl.o_waug);
   c.w_augs = at<void>(ws, pl.o_waugs);
+  return c;
+}
+int run_coop(const Plan& pl, const void* x, void* ws, hipStream_t s) {
+  if (pl.D == 128 && pl.cG > 1 && (uintptr_t)x % 16 != 0)
+    return fail(GMMXX_ERR_INVALID_ARGUMENT, "x must be 16-byte aligned for spherical bf16 at D = 128");
+  CoopArgs c = sb_args(pl, x, ws);
+  c.w_aug = at<void>(ws, pl.o_waug);
   c.G = pl.cG;
   c.NG = pl.cNG;
   c.spb = pl.cspb;
@@ -581,9 +588,9 @@ int prepare(const Plan& pl, const void* x, const float* means, const float* covs
   a.w_hi = at<void>(ws, pl.o_whi);
   a.w_lo = pl.bf ? at<void>(ws, pl.o_wlo) : nullptr;
   a.w_aug = (pl.bf && pl.cov == SPH) ? at<void>(ws, pl.o_waug) : nullptr;
-  a.w_mu = (pl.coop || pl.fused) ? at<void>(ws, pl.o_wmu) : nullptr;
-  a.w_scale = (pl.coop || pl.fused) ? at<float>(ws, pl.o_wsc) : nullptr;
-  a.w_augs = (pl.fused || (pl.coop && pl.cG == 1)) ? at<void>(ws, pl.o_waugs) : nullptr;
+  a.w_mu = pl.sb ? at<void>(ws, pl.o_wmu) : nullptr;
+  a.w_scale = pl.sb ? at<float>(ws, pl.o_wsc) : nullptr;
+  a.w_augs = pl.sb ? at<void>(ws, pl.o_waugs) : nullptr;
   a.cconst = at<float4>(ws, pl.o_cconst);
   a.gram = shift ? gram : nullptr;
   a.shift = gram ? shift : nullptr;
@@ -599,6 +606,11 @@ int prepare(const Plan& pl, const void* x, const float* means, const float* covs
 int lse_pass(const Plan& pl, const void* x, void* ws, float* scores, int64_t* labels, bool with_ll,
              hipStream_t s) {
   const bool only = labels && !scores && !with_ll;
+  if (only && pl.sb) {
+    if (launch_sph_bf16_label(round_up(pl.D, 32), sb_args(pl, x, ws), labels, s) != 0)
+      return fail(GMMXX_ERR_UNSUPPORTED, "no label kernel for this shape");
+    return check_hip("label pass");
+  }
   TileArgs t = tile_args(pl, x, ws, /*em=*/only);
   const bool direct = only && pl.ktiles == 1;
   if (direct) t.labels = labels;

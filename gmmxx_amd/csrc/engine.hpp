@@ -100,6 +100,9 @@ int coop_capacity(int dp, int G, bool exact);
 int launch_sph_bf16_coop(int dp, const CoopArgs& a, hipStream_t s);
 // (a.G, a.xch and a.status unused; a.NG workgroups)
 int launch_sph_bf16_one(int dp, int nw, const CoopArgs& a, hipStream_t s);
+// Labels of spherical bf16 rows, K <= 1024 (em_label.hip; x, vec, N, D, K, B, DL, w_mu,
+// w_scale and w_augs of a are read).
+int launch_sph_bf16_label(int dp, const CoopArgs& a, int64_t* labels, hipStream_t s);
 
 // Full covariance at 16 < D <= 128 (em_full_wide.hip): whitening E-step and
 // weighted-Gram statistics on split-bf16 MFMA operands (the statistics at DP = 128

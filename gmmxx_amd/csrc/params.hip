@@ -149,7 +149,10 @@ __global__ __launch_bounds__(64) void prep_kernel(PrepArgs a) {
         }
 #pragma unroll
         for (int off = 32; off >= 1; off /= 2) mb64 += __shfl_xor(mb64, off);
-        const double cp = -0.5 * mb64 + ((double)lw - 0.5 * (double)D * (kLog2Pi + log((double)var))) * (double)var;
+        double cp = -0.5 * mb64 + ((double)lw - 0.5 * (double)D * (kLog2Pi + log((double)var))) * (double)var;
+        // A weight of zero: l2 about -1e30, finite in all three parts (the remainders of an
+        // infinite one are NaN).
+        if (lw == -INFINITY) cp = -1e30 * fmin((double)var, 1e8);
         const __bf16 ph = (__bf16)(float)cp;
         const __bf16 pm = (__bf16)(float)(cp - (double)(float)ph);
         const __bf16 pl = (__bf16)(float)(cp - (double)(float)ph - (double)(float)pm);
