@@ -310,7 +310,7 @@ int plan_problem(const gmmxx_problem* p, Plan* pl) {
   q.o_lpaug = take(q.fw ? BK * (q.DP / 32) * 64 * 8 * 2 : 0);
   q.o_l2w = take(q.fw ? BK * (size_t)q.N * 4 : 0);
   q.o_linv = take((q.fw || q.w16) ? BK * q.D * q.D * 4 : 0);
-  q.o_w16parts = take(q.w16 ? BK * 3 * 512 * 2 : 0);   // three 1 KB MFMA operands per component
+  q.o_w16parts = take(q.w16 ? BK * 3 * 256 * 2 : 0);   // three 16 x 16 bf16 parts per component
   q.o_w16b = take(q.w16 ? BK * 16 * 4 : 0);
   q.o_w16c = take(q.w16 ? BK * 4 : 0);
   q.total = off;

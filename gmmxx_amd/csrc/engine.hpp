@@ -174,11 +174,10 @@ struct Full16Args {
   const float* means;
   const float* weights;
   const float* logdet;
-  void* lparts;                // [B][K][3][16][16] bf16 parts of L^-1
+  void* lparts;                // [B][K][3][2][16][8] bf16 parts of L^-1
   float* bneg;                 // [B][K][16] -L^-1 μ
   float* c2;                   // [B][K] log2 w - ½ log2(e) (D log 2π + log det)
   float* scores;               // [B][N] natural-log scores, or null
-  float* lse2;                 // [B][N] log2 log-normalisers, or null
   int64_t* labels;             // [B][N] first argmax, or null
   float* proba;                // [B][N][K] responsibilities, or null
 };
