@@ -271,7 +271,9 @@ def single_pass(cfg):
 def kernel_label(cfg, phase):
     """Name of the kernel that runs in `phase` for this config (see gmmxx_amd/csrc)."""
     if cfg["cov"] == "full" and cfg["D"] > 16:
-        return "fw_estep_kernel" if phase == "lse_tile" else "fw_stats_kernel"
+        if phase == "lse_tile":
+            return "fw_estep_kernel"
+        return "fw_stats_tile_kernel" if cfg["K"] > 8 else "fw_stats_kernel"
     one = single_pass(cfg)
     if one:
         return f"{one} (single pass)"

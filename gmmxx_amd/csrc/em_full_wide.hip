@@ -27,7 +27,8 @@
 //                    squares of its 16 entries; the partner lane (l ^ 32) holds the
 //                    other 16.  The row's log-normaliser is accumulated online over
 //                    the components; the log2 logits go to a (B, K, N) buffer;
-//   fw_stats_kernel  one wave per component and row slice (D = 128:
+//   fw_stats_kernel  (K <= 8 and where 16-component workgroups would mostly pad; else
+//                    em_full_stats.hip) one wave per component and row slice (D = 128:
 //                    fw_stats128_kernel, two waves of five tiles each):
 //                    Σ_n r_n x_n x_nᵀ = Σ w wᵀ with w = √r·x as the lower 32 x 32
 //                    tiles over 16-row k-steps, one split of w serving as both
