@@ -66,8 +66,7 @@ __global__ __launch_bounds__(64 * NW, 2) void sph_bf16_one_kernel(CoopArgs a) {
   const int K = a.K, D = EXACT ? DP : a.D;
   const int kbase = wave * kCW;
 
-  // Staged rows start at zero (the lead-in M-GEMM multiplies r = 0 by them), with
-  // the constant augmented columns 8..31: [1 0 0 ...].
+  // Staged rows start at zero, with the constant augmented columns 8..31: [1 0 0 ...].
   for (int i = tid; i < kNB * kBN * XS / 8; i += NTHR) *reinterpret_cast<uint4*>(xs + 8 * i) = make_uint4(0, 0, 0, 0);
   __syncthreads();
   for (int i = tid; i < kNB * kBN; i += NTHR) xs[i * XS + DP + 8] = (__bf16)1.f;
@@ -170,8 +169,10 @@ __global__ __launch_bounds__(64 * NW, 2) void sph_bf16_one_kernel(CoopArgs a) {
     __syncthreads();
 
     // i = 0 .. nblk: the E-GEMM of block i (i = nblk: a stale buffer, discarded)
-    // and the M-GEMM of block i-1 (i = 0: r = 0).
-    int bufE = 0, bufM = kNB - 1;
+    // and the M-GEMM of block i-1.  i = 0 multiplies r = 0 by the item's own first
+    // block: another buffer may hold rows of the previous item, and 0 · NaN of one that
+    // is not finite would reach this problem's sums.
+    int bufE = 0, bufM = 0;
     for (int i = 0; i <= nblk; ++i) {
       const int pb = i & 1;
       const int bufN = bufE + 1 == kNB ? 0 : bufE + 1;     // buffer of block i+1 (== of block i-2)

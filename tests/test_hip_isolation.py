@@ -1,0 +1,44 @@
+"""Problems of one call stay apart where a workgroup of the single-pass spherical bf16
+kernels takes a second one (more problems than workgroups or groups): rows of
+problem 0 that are not finite leave every other problem's statistics bit-equal, and
+the later problems match the oracle (bf16 bar of test_hip_parity: 2e-3 of the
+statistic's scale)."""
+
+import pytest
+import torch
+
+from oracle import torch_ref
+from tests.test_hip_parity import make_problem, to_dev
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+# (B, N, D, K): one workgroup per problem of two, four and eight waves (1024, 512 and 256
+# workgroups), three row blocks (the staging's buffer count)
+ONE = [(1100, 96, 72, 50), (600, 96, 121, 60), (600, 96, 72, 100), (300, 96, 72, 200), (300, 96, 128, 256)]
+
+
+def _stats(hip, x, p):
+    return [t.cpu() for t in hip.estep_stats("spherical", x, *p)[:3]]
+
+
+def _check(hip, b, n, d, k, bad_rows):
+    x, means, covs, w = make_problem("spherical", b, n, d, k, seed=97, dtype=BF)
+    p = [to_dev(t) for t in (means, covs, w)]
+    good = _stats(hip, to_dev(x, BF), p)
+    last = [t[-8:] for t in (x, means, covs, w)]
+    for got, exp in zip(good, torch_ref.estep_stats(last[0], "spherical", *last[1:])):
+        torch.testing.assert_close(got[-8:], exp, rtol=2e-3, atol=2e-3 * max(1e-30, float(exp.abs().max())))
+    for value in (float("nan"), float("inf"), 1e30):      # (1e30: ‖x‖² overflows)
+        bad = x.clone()
+        for row in bad_rows:
+            bad[0, row, row % d] = value
+        got = _stats(hip, to_dev(bad, BF), p)
+        for a, e in zip(got, good):
+            assert torch.equal(a[1:], e[1:]), f"{value} in problem 0 reached another problem"
+
+
+@pytest.mark.parametrize("b,n,d,k", ONE, ids=[f"B{c[0]}-D{c[2]}-K{c[3]}" for c in ONE])
+def test_one_workgroup_per_problem(hip, b, n, d, k):
+    print(f"[isolation] B={b} N={n} D={d} K={k}", flush=True)
+    _check(hip, b, n, d, k, (3, 40, 70, 95))
