@@ -131,8 +131,8 @@ __global__ __launch_bounds__(64 * kNW) void sph_bf16_coop_kernel(CoopArgs a) {
   const int kbase = mem * (kNW * kCW) + __builtin_amdgcn_readfirstlane(wave) * kCW;
   uint64_t* const gxch = a.xch + (size_t)grp * kRing * G * kBN;
 
-  // Staged rows start at zero: the lead-in blocks multiply r = 0 by buffers no
-  // block has filled yet, which must not hold NaN bit patterns.
+  // Staged rows start at zero: the lead-in and drain blocks multiply r = 0 by buffers
+  // no block has filled yet, which must not hold NaN bit patterns.
   for (int i = tid; i < kNB * kBN * XS / 8; i += NTHR) *reinterpret_cast<uint4*>(xs + 8 * i) = make_uint4(0, 0, 0, 0);
   __syncthreads();
   // Constant augmented columns 8..31 of every staged row: [1 0 0 ...].
@@ -335,6 +335,17 @@ __global__ __launch_bounds__(64 * kNW) void sph_bf16_coop_kernel(CoopArgs a) {
       red_m[(pb * kNW + wave) * RR + lr] = m;
       red_s[(pb * kNW + wave) * RR + lr] = sum;
     };
+    if (seq != 0) {
+      // The buffers hold the previous item's rows: 0 · NaN of one that is not finite would
+      // reach this problem's sums.  (Reading the item's own first block there instead, by a
+      // choice of buffer in the loop, cost 1.7 % at N = 1M, D = 64, K = 1000.)
+      constexpr int CH = DP / 8 + 1;              // x, and the augmented columns 0..7
+      int t = tid;
+      unsigned z = 0;
+      asm volatile("" : "+v"(t), "+v"(z));        // (formed here, not kept in registers)
+      for (; t < kNB * kBN * CH; t += NTHR) *reinterpret_cast<uint4*>(xs + t / CH * XS + 8 * (t % CH)) = make_uint4(z, z, z, z);
+      __syncthreads();
+    }
     if (nblk > 0) { fetch(0); stash(0); }
     if (nblk > 1) { fetch(kBN); stash(1); }
     if (nblk > 2) fetch(2 * kBN);
@@ -343,10 +354,9 @@ __global__ __launch_bounds__(64 * kNW) void sph_bf16_coop_kernel(CoopArgs a) {
     // Iteration i of the block pipeline, i = 0 .. nblk + 1 (rounded up to even):
     // the E-GEMM of block i and the M-GEMM of block i-2.  Every iteration runs
     // the same code: the lead-in blocks -2, -1 and the drain blocks nblk,
-    // nblk + 1 compute on zeroed or stale staged rows (in bounds) and add
-    // nothing, since their rows get r = 0 and take part in no exchange and no
-    // log-likelihood.  PB = i & 1, the LDS/register slot parity of blocks i
-    // and i-2.
+    // nblk + 1 compute on rows of this item or zeros and add nothing, since their
+    // rows get r = 0 and take part in no exchange and no log-likelihood.
+    // PB = i & 1, the LDS/register slot parity of blocks i and i-2.
 #pragma unroll
     for (int pb = 0; pb < 2; ++pb) {
 #pragma unroll

@@ -16,6 +16,9 @@ BF = torch.bfloat16
 # (B, N, D, K): one workgroup per problem of two, four and eight waves (1024, 512 and 256
 # workgroups), three row blocks (the staging's buffer count)
 ONE = [(1100, 96, 72, 50), (600, 96, 121, 60), (600, 96, 72, 100), (300, 96, 72, 200), (300, 96, 128, 256)]
+# groups of two, three and four workgroups (128, 80 and 64 groups of the 256 resident
+# workgroups), five row blocks and more
+GROUPS = [(160, 160, 40, 300), (160, 200, 96, 300), (100, 160, 128, 600), (80, 161, 121, 900)]
 
 
 def _stats(hip, x, p):
@@ -42,3 +45,9 @@ def _check(hip, b, n, d, k, bad_rows):
 def test_one_workgroup_per_problem(hip, b, n, d, k):
     print(f"[isolation] B={b} N={n} D={d} K={k}", flush=True)
     _check(hip, b, n, d, k, (3, 40, 70, 95))
+
+
+@pytest.mark.parametrize("b,n,d,k", GROUPS, ids=[f"B{c[0]}-D{c[2]}-K{c[3]}" for c in GROUPS])
+def test_one_group_per_problem(hip, b, n, d, k):
+    print(f"[isolation] B={b} N={n} D={d} K={k}", flush=True)
+    _check(hip, b, n, d, k, (3, 40, 70, 100, 130, n - 1))
