@@ -619,6 +619,7 @@ int lse_pass(const Plan& pl, const void* x, void* ws, float* scores, int64_t* la
   if (direct) return check_hip("label pass");
   CombineArgs c{};
   c.B = pl.B;
+  c.K = pl.K;
   c.ktiles = labels ? pl.ktiles : pl.lktiles;
   c.N = pl.N;
   c.part_ms = t.part_ms;
@@ -845,6 +846,7 @@ int gmmxx_hip_em_phase(const gmmxx_problem* p, int phase, const void* x, float* 
       if (ll_in_pass(pl)) return GMMXX_OK;
       CombineArgs c{};
       c.B = pl.B;
+      c.K = pl.K;
       c.ktiles = pl.lktiles;
       c.N = pl.N;
       c.part_ms = at<float>(ws, pl.o_pms);
@@ -1061,6 +1063,7 @@ int gmmxx_hip_estep_stats_topk(const gmmxx_problem* p, const void* x, const floa
     if (run_tile(pl, MODE_IDX, t, s) != 0) return fail(GMMXX_ERR_UNSUPPORTED, "no tile kernel for this shape");
     CombineArgs c{};
     c.B = pl.B;
+    c.K = pl.K;
     c.ktiles = pl.ktiles;
     c.N = pl.N;
     c.part_ms = t.part_ms;

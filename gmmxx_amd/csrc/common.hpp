@@ -95,6 +95,10 @@ __device__ __forceinline__ uint4 ld16_any(const void* p) {
   return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
+// The label of a row whose first maximum is component idx: 0 where none of the K components
+// has it (a row of NaN, as torch.argmax gives; logits below the padding components').
+__device__ __forceinline__ int64_t label_of(int idx, int K) { return (unsigned)idx < (unsigned)K ? idx : 0; }
+
 // Merge two (max, scaled-sum, argmax) triples; ties keep the smaller index.
 __device__ __forceinline__ void lse_merge(float& m, float& s, int& idx, float m2, float s2, int i2) {
   float M = fmaxf(m, m2);

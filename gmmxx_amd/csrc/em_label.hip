@@ -8,7 +8,8 @@
 // covers 256 components per workgroup).  An x operand read from LDS serves all CT tiles;
 // the scales stay in LDS.  Per row: the maximum over the lane's 16·CT logits, its first
 // place, the partner lane (l ^ 32), then the waves through LDS one block later; equal
-// maxima take the lower component.
+// maxima take the lower component.  Padding components and those of weight zero are
+// -inf, so no finite row is far enough out to be labelled with one.
 //
 // Bound: at K <= 64 the latency of the reads of x (1M x 32, K = 64: 2.6 TB/s with the
 // labels); with more components the 16·CT multiplies, maxima and compares per row and
@@ -72,7 +73,7 @@ __global__ __launch_bounds__(64 * NW, CT == 1 ? 4 : 2) void sph_bf16_label_kerne
       for (int e = 0; e < 8; ++e) {
 #pragma unroll
         for (int t = 0; t < XK; ++t) wmu[ct][t][e] = (__bf16)0.f;
-        waug[ct][e] = (__bf16)((8 * hf + e) == 6 ? -kHuge : 0.f);
+        waug[ct][e] = (__bf16)((8 * hf + e) == 6 ? -INFINITY : 0.f);   // (below every row's logits)
       }
     }
   }
@@ -126,7 +127,7 @@ __global__ __launch_bounds__(64 * NW, CT == 1 ? 4 : 2) void sph_bf16_label_kerne
       if constexpr (NW >= 2) low(__builtin_amdgcn_update_dpp(0, idx, 0xB1, 0xF, 0xF, false));
       if constexpr (NW >= 4) low(__builtin_amdgcn_update_dpp(0, idx, 0x4E, 0xF, 0xF, false));
       if constexpr (NW >= 8) low(__builtin_amdgcn_update_dpp(0, idx, 0x141, 0xF, 0xF, false));
-      if (w == 0 && r0 + r < nrows) labels[(size_t)b * N + rbeg + r0 + r] = (int64_t)idx;
+      if (w == 0 && r0 + r < nrows) labels[(size_t)b * N + rbeg + r0 + r] = label_of(idx, K);
     }
   };
 

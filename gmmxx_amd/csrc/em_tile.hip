@@ -631,7 +631,7 @@ __global__ __launch_bounds__(512) void em_tile_kernel(TileArgs a) {
       }
       const int64_t n = n0 + r;
       if (MODE == MODE_IDX && a.labels) {       // (uniform) every component is in this workgroup
-        if (w == 0 && n < rend) a.labels[(size_t)b * N + n] = (int64_t)idx;
+        if (w == 0 && n < rend) a.labels[(size_t)b * N + n] = label_of(idx, K);
       } else if (w == 0 && n < rend) {
         const size_t og = ((size_t)ktile * a.B + b) * N + n;
         reinterpret_cast<float2*>(a.part_ms)[og] = make_float2(M, t);

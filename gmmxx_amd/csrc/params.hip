@@ -149,14 +149,14 @@ __global__ __launch_bounds__(64) void prep_kernel(PrepArgs a) {
         }
 #pragma unroll
         for (int off = 32; off >= 1; off /= 2) mb64 += __shfl_xor(mb64, off);
-        double cp = -0.5 * mb64 + ((double)lw - 0.5 * (double)D * (kLog2Pi + log((double)var))) * (double)var;
-        // A weight of zero: l2 about -1e30, finite in all three parts (the remainders of an
-        // infinite one are NaN).
-        if (lw == -INFINITY) cp = -1e30 * fmin((double)var, 1e8);
-        const __bf16 ph = (__bf16)(float)cp;
-        const __bf16 pm = (__bf16)(float)(cp - (double)(float)ph);
-        const __bf16 pl = (__bf16)(float)(cp - (double)(float)ph - (double)(float)pm);
+        const double cp = -0.5 * mb64 + ((double)lw - 0.5 * (double)D * (kLog2Pi + log((double)var))) * (double)var;
+        // A weight of zero (inference only) is -inf in the first part alone: the remainders
+        // of an infinite C' would be NaN.
+        const bool none = lw == -INFINITY;
         const __bf16 half = (__bf16)(-0.5f), zero = (__bf16)0.f;
+        const __bf16 ph = (__bf16)(none ? -INFINITY : (float)cp);
+        const __bf16 pm = none ? zero : (__bf16)(float)(cp - (double)(float)ph);
+        const __bf16 pl = none ? zero : (__bf16)(float)(cp - (double)(float)ph - (double)(float)pm);
         const __bf16 vals[9] = {half, half, half, zero, zero, zero, ph, pm, pl};
         if (lane < 16) reinterpret_cast<__bf16*>(a.w_augs)[bk * 16 + lane] = lane < 9 ? vals[lane] : zero;
       }
@@ -855,7 +855,7 @@ __global__ void combine_kernel(CombineArgs a) {
     if (a.lse2) a.lse2[o] = lse2;
     const float lse = lse2 * kLn2;
     if (a.scores) a.scores[o] = lse;
-    if (a.labels) a.labels[o] = (int64_t)idx;
+    if (a.labels) a.labels[o] = label_of(idx, a.K);
     if (a.idx32) a.idx32[o] = idx;
     contrib = (double)lse;
   }

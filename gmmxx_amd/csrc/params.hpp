@@ -31,7 +31,7 @@ struct PrepArgs {
 };
 
 struct CombineArgs {
-  int B, ktiles;
+  int B, K, ktiles;
   int64_t N;
   const float* part_ms;
   const int* part_idx;

@@ -231,7 +231,8 @@ int gmmxx_hip_finalize_stats(const gmmxx_problem* p, const float* nk, const floa
                              void* stream);
 
 /* Inference under fixed parameters (no prelude): per-sample log-likelihood
- * `scores` (B, N) and/or first-maximum labels (B, N) int64; either may be NULL.
+ * `scores` (B, N) and/or first-maximum labels (B, N) int64, each in [0, K) (0 for a
+ * row without a maximum, as one of NaN); either may be NULL.
  * Replaces spherical/diag/full assign + logsumexp (gmmxx/csrc/bindings.cpp:19-58,
  * :140-190; gmmxx/_cuda.py:1246-1314) and the torch inference functions
  * *_assign_torch_native_chunked / *_score_samples_torch_native_chunked
