@@ -413,7 +413,12 @@ int run_coop(const Plan& pl, const void* x, void* ws, hipStream_t s) {
   c.status = at<unsigned>(ws, pl.o_flags);
   // Polls per wait before the pass gives up; GMMXX_HIP_COOP_SPIN_LIMIT overrides
   // it (a negative value gives up at the first wait: the timeout path, on demand).
-  c.spin_limit = 1 << 20;
+  // An XCD starts its workgroups in id order, so at most one group per XCD has members
+  // still to start, and they get the next compute unit that any kernel leaves: a wait ends
+  // with the kernels that share the GPU, and the limit (tens of seconds; a poll is a sleep of
+  // 64 cycles and an L2 load) is there for what never ends.  At 2^20 polls, under a second,
+  // a fit beside a long kernel of another stream could fail where it only has to wait.
+  c.spin_limit = 1 << 26;
   if (const char* sl = getenv("GMMXX_HIP_COOP_SPIN_LIMIT")) c.spin_limit = atoi(sl);
   const int rc = pl.cG == 1 ? launch_sph_bf16_one(pl.cDP, pl.cnw, c, s) : launch_sph_bf16_coop(pl.cDP, c, s);
   if (rc == -2) return fail(GMMXX_ERR_HIP, "launch of the single-pass cooperative kernel failed");
@@ -427,7 +432,7 @@ int run_xch(const Plan& pl, const void* x, void* ws, hipStream_t s, bool em = tr
   t.rows_per_slice = pl.xrows;
   t.xch = at<uint64_t>(ws, pl.o_xch);
   t.status = at<unsigned>(ws, pl.o_flags);
-  t.spin_limit = 1 << 20;   // as the cooperative pass (GMMXX_HIP_COOP_SPIN_LIMIT overrides)
+  t.spin_limit = 1 << 20;   // polls per wait, as the cooperative pass's (GMMXX_HIP_COOP_SPIN_LIMIT overrides)
   if (const char* sl = getenv("GMMXX_HIP_COOP_SPIN_LIMIT")) t.spin_limit = atoi(sl);
   const int64_t nwords = (int64_t)pl.B * pl.xslices * kRing * pl.ktiles * kBN;
   const int rc = launch_tile_xch(pl.cov, pl.DP, t, dim3(pl.xslices * pl.ktiles, pl.B), nwords, s);
