@@ -379,14 +379,30 @@ __global__ __launch_bounds__(512) void em_tile_kernel(TileArgs a) {
   // the pass lost 5 % to loading by element).  Label pass at N = 1M, D = 100,
   // K = 500: 0.84 -> 0.65 ms with the exponentials gone too; the 32-bit offsets also
   // took the C3 exchange pass from 29 spilled VGPRs to 20 (30.9 -> 30.4 ms a fit).
+  // BYELEM: the exchange pass at DP <= 32 loads rows that are not whole aligned chunks by
+  // element, masked in the fetch: there the loads wait beside the exchange, and the
+  // masks and shifts of `settle` would sit in a loop bound by VALU issue (ten iterations,
+  // settled -> by element: spherical 200k x 6, K = 400 2023 -> 1924 us; 400k x 21, K = 705
+  // 5858 -> 5573; diag 200k x 6, K = 400 2047 -> 1952; tied 200k x 9, K = 900 4070 -> 3833; at
+  // DP = 64 settled is the faster form: spherical 200k x 50, K = 600 3736 against 3796).
+  constexpr bool BYELEM = XCH && DP <= 32;
   auto rows_left = [&](int64_t n0) -> int { return rend - n0 < kBN ? (int)(rend - n0) : kBN; };
   auto load_chunk = [&](int c, int64_t n0, int left) -> uint4 {
     const int r = c / CPR, cc = (c % CPR) * VEC;
     const XT* blk = xb + (size_t)n0 * D;
+    if constexpr (BYELEM) {
+      if (r >= left) return make_uint4(0, 0, 0, 0);
+      if (a.vec_ok) return *reinterpret_cast<const uint4*>(blk + r * D + cc);
+      union { uint4 u; XT e[VEC]; } t;
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) t.e[j] = (cc + j < D) ? blk[r * D + cc + j] : (XT)0.f;
+      return t.u;
+    }
     const int row = (r < left ? r : left - 1) * D;
     return ld16_any(blk + (row + (cc < D - VEC ? cc : D - VEC)));
   };
   auto settle = [&](uint4 raw, int cc, int r, int left) -> uint4 {
+    if constexpr (BYELEM) return raw;
     if (D < DP) {                            // (uniform) columns past the row's end are zero
       if constexpr (!BF) {
         if (D % VEC && D > VEC) {
@@ -403,7 +419,7 @@ __global__ __launch_bounds__(512) void em_tile_kernel(TileArgs a) {
   };
   // Rows shorter than one load (16 bytes could pass the end of x) are read by element
   // when they are staged.
-  const bool narrow = DP <= 16 && D < VEC;   // (uniform)
+  const bool narrow = !BYELEM && DP <= 16 && D < VEC;   // (uniform)
   auto load_narrow = [&](int c, int64_t n0, int left) -> uint4 {
     const int r = c / CPR, cc = (c % CPR) * VEC;
     const XT* row = xb + (size_t)(n0 + (r < left ? r : left - 1)) * D;

@@ -8,7 +8,7 @@ namespace gx {
 
 struct TileArgs {
   const void* x;               // [B][N][D], fp32 or bf16
-  int vec_ok;                  // bf16: x rows are 16-byte aligned and D == DP
+  int vec_ok;                  // x rows are 16-byte aligned and D == DP (bf16, and fp32 XCH at DP <= 32)
   int64_t N;
   int D, K, B;
   int ktiles;                  // component tiles per batch

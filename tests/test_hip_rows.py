@@ -64,3 +64,27 @@ def test_rows_off_a_16_byte_boundary(hip, cov):
         ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
     assert rc == 0, hip.last_error()
     assert_labels(labels, x, means, covs, w, cov, 1e-5)
+
+
+@pytest.mark.parametrize("cov,d,k", [("spherical", 3, 300), ("spherical", 16, 600), ("spherical", 32, 300),
+                                     ("diag", 21, 300), ("tied", 32, 900), ("spherical", 64, 300)])
+def test_exchange_rows_off_a_16_byte_boundary(hip, cov, d, k):
+    """Several component tiles: the statistics of rows at any element address are those of
+    the same rows on a boundary (which D = 16 and 32 read whole), bit for bit."""
+    import ctypes
+    n = 1000
+    x, means, covs, w = make_problem(cov, 1, n, d, k, seed=83)
+    xd = to_dev(x)
+    p = [to_dev(t) for t in (means, covs, w)]
+    exp = hip.estep_stats(cov, xd, *p)
+    xu = _unaligned(xd)
+    prob = hip.problem(cov, torch.float32, 1, n, d, k)
+    ws = hip.Workspace(prob, xd.device)
+    got = [None if t is None else torch.empty_like(t) for t in exp]
+    ptr = lambda t: None if t is None else ctypes.c_void_p(t.data_ptr())      # noqa: E731
+    rc = hip.load_library().gmmxx_hip_estep_stats(
+        ctypes.byref(prob), ptr(xu), *map(ptr, p), 1e-6, 1e-8, *map(ptr, got), ws.ptr, ws.nbytes,
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0, hip.last_error()
+    for a, e in zip(got, exp):
+        assert e is None or torch.equal(a, e)
