@@ -57,6 +57,7 @@ struct Plan {
   int cDP = 0, cnw = 0;      // coop: padded row width, waves per workgroup
   int cG = 0, cNG = 0, cspb = 0;   // coop: workgroups per group, groups, row items per batch
   int64_t crows = 0;         // coop: rows per item
+  bool short_slices = false; // one row block per slice: the slice sums are added in double
   int fslices = 0;           // fused: one wave per row slice
   int fparts = 0;            // fused: partial results (one per workgroup of kFusedWaves slices)
   int64_t frows = 0;
@@ -161,9 +162,11 @@ int plan_problem(const gmmxx_problem* p, Plan* pl) {
   const int64_t row_blocks = (q.N + kBN - 1) / kBN;
   const int64_t target_blocks = (kTargetWaves + q.nw - 1) / q.nw;
   int64_t slices = std::max<int64_t>(1, (target_blocks + (int64_t)q.ktiles * q.B - 1) / ((int64_t)q.ktiles * q.B));
-  // (problems that leave most CUs idle: one block per slice, the shortest chain)
-  const int64_t min_blocks = row_blocks * q.ktiles * q.B <= 256 ? 1 : kMinBlocksPerSlice;
-  slices = std::min(slices, std::max<int64_t>(1, row_blocks / min_blocks));
+  // Problems that leave most CUs idle: one block per slice, the shortest chain.  Their sums
+  // are added in double: in fp32 the statistics of 800 rows were 1.2 to 1.9 times as far
+  // from float64 as with three blocks per slice.
+  q.short_slices = row_blocks * q.ktiles * q.B <= 256;
+  slices = std::min(slices, std::max<int64_t>(1, row_blocks / (q.short_slices ? 1 : kMinBlocksPerSlice)));
   q.rows_per_slice = ((q.N + slices - 1) / slices + kBN - 1) / kBN * kBN;
   q.slices = (int)((q.N + q.rows_per_slice - 1) / q.rows_per_slice);
   q.cblocks = combine_blocks(q.N);
@@ -461,6 +464,8 @@ LlFold ll_fold(const Plan& pl, void* ws, int parts, double inv_total, float* out
 int stat_slices(const Plan& pl) {
   return pl.fw ? pl.fw_slices : (pl.fused ? pl.fparts : (pl.coop ? pl.cspb : (pl.xch ? pl.xslices : pl.slices)));
 }
+// Whether the partial sums are those of one-block slices (the tile pass's own).
+bool wide_sums(const Plan& pl) { return pl.short_slices && !(pl.fw || pl.fused || pl.coop || pl.xch); }
 // The tile-partial buffer is free once the statistics are being reduced: it is
 // the scratch of the grouped slice reduction.
 float* red_tmp(const Plan& pl, void* ws) { return at<float>(ws, pl.o_pms); }
@@ -643,7 +648,7 @@ int stats_pass(const Plan& pl, const void* x, void* ws, hipStream_t s) {
   if (run_tile(pl, MODE_STATS, t, s) != 0)
     return fail(GMMXX_ERR_UNSUPPORTED, "no tile kernel for this shape");
   launch_reduce_slices(t.part_stats, pl.slices, (int64_t)pl.B * pl.K * pl.JP, at<float>(ws, pl.o_stats), s,
-                       red_tmp(pl, ws), red_tmp_floats(pl));
+                       red_tmp(pl, ws), red_tmp_floats(pl), nullptr, pl.short_slices);
   return check_hip("statistics pass");
 }
 
@@ -881,7 +886,7 @@ int gmmxx_hip_em_phase(const gmmxx_problem* p, int phase, const void* x, float* 
       }
       launch_reduce_slices(at<float>(ws, pl.o_pstats), stat_slices(pl), (int64_t)pl.B * pl.K * pl.JP,
                            at<float>(ws, pl.o_stats), s, red_tmp(pl, ws), red_tmp_floats(pl),
-                           ll_in_pass(pl) ? &ll : nullptr);
+                           ll_in_pass(pl) ? &ll : nullptr, wide_sums(pl));
       return check_hip("statistics reduction");
     }
     case GMMXX_PHASE_FINALIZE:
@@ -917,7 +922,7 @@ int gmmxx_hip_em_step(const gmmxx_problem* p, const void* x, float* means, float
   if (tied_shift(pl, ws)) parts += pl.B * pl.D;   // -½ tr(P XᵀX) rows, from the prepare phase
   launch_reduce_finalize(f, at<float>(ws, pl.o_pstats), stat_slices(pl), red_tmp(pl, ws), red_tmp_floats(pl),
                          ll_fold(pl, ws, parts, 1.0 / ((double)pl.B * (double)pl.N), lower_bound),
-                         (hipStream_t)stream);
+                         (hipStream_t)stream, wide_sums(pl));
   return check_hip("reduction and finalize");
 }
 
@@ -973,7 +978,7 @@ int gmmxx_hip_estep_stats(const gmmxx_problem* p, const void* x, const float* me
     }
     const LlFold ll = ll_fold(pl, ws, ll_parts(pl), 1.0, ll_sum);
     launch_reduce_slices(at<float>(ws, pl.o_pstats), stat_slices(pl), (int64_t)pl.B * pl.K * pl.JP,
-                         at<float>(ws, pl.o_stats), s, red_tmp(pl, ws), red_tmp_floats(pl), &ll);
+                         at<float>(ws, pl.o_stats), s, red_tmp(pl, ws), red_tmp_floats(pl), &ll, wide_sums(pl));
     if ((rc = check_hip("fused statistics pass"))) return rc;
   } else {
     if ((rc = lse_pass(pl, x, ws, nullptr, nullptr, true, s))) return rc;
@@ -1090,7 +1095,7 @@ int gmmxx_hip_estep_stats_topk(const gmmxx_problem* p, const void* x, const floa
     ll.inv_total = 1.0;
     ll.out = ll_sum;
     launch_reduce_slices(u.part_stats, pl.slices, (int64_t)pl.B * pl.K * pl.JP, at<float>(ws, pl.o_stats), s,
-                         red_tmp(pl, ws), red_tmp_floats(pl), &ll);
+                         red_tmp(pl, ws), red_tmp_floats(pl), &ll, pl.short_slices);
   } else {
   if (pl.bf && pl.cov == SPH && pl.DP >= 128) {
     if ((rc = lse_pass(pl, x, ws, nullptr, nullptr, false, s))) return rc;
@@ -1108,7 +1113,7 @@ int gmmxx_hip_estep_stats_topk(const gmmxx_problem* p, const void* x, const floa
   u.thr_idx = thri;
   if (run_tile(pl, MODE_STATS_TOPK, u, s) != 0) return fail(GMMXX_ERR_UNSUPPORTED, "no tile kernel for this shape");
   launch_reduce_slices(u.part_stats, pl.slices, (int64_t)pl.B * pl.K * pl.JP, at<float>(ws, pl.o_stats), s,
-                       red_tmp(pl, ws), red_tmp_floats(pl));
+                       red_tmp(pl, ws), red_tmp_floats(pl), nullptr, pl.short_slices);
   launch_ll_reduce(tll, pl.B * sel_blocks, 1.0, ll_sum, s);
   }
   if ((rc = check_hip("approximate top-k statistics"))) return rc;

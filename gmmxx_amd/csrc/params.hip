@@ -1005,14 +1005,15 @@ __global__ void ll_reduce_kernel(const double* ll_part, int count, double inv_to
 
 // out[i] = Σ_s part[s * M + i] in a fixed order (deterministic): a block owns
 // 64 outputs; wave g sums slices g, g + 16, ...; the 16 wave sums are then
-// added in wave order.
+// added in wave order.  ACC: the type of the sums (launch_reduce_slices).
 constexpr int kRedWaves = 16;
 // blockIdx.y selects a group of `per` consecutive slices (written to out + y*M).
 // ll.out != null: the grid has one more workgroup (the last), which does the
 // log-likelihood reduction of LlFold instead.
+template <typename ACC>
 __global__ __launch_bounds__(64 * kRedWaves) void reduce_slices_kernel(const float* part, int slices, int64_t M,
                                                                        float* out, int per, LlFold ll) {
-  __shared__ float red[kRedWaves][64];
+  __shared__ ACC red[kRedWaves][64];
   if (ll.out && blockIdx.x == gridDim.x - 1) {
     __shared__ double scratch[32];
     double t = 0.0;
@@ -1033,15 +1034,15 @@ __global__ __launch_bounds__(64 * kRedWaves) void reduce_slices_kernel(const flo
   part += (size_t)blockIdx.y * per * M;
   out += (size_t)blockIdx.y * M;
   slices = min(per, slices - (int)blockIdx.y * per);
-  float s = 0.f;
+  ACC s = 0;
   if (i < M)
     for (int t = g; t < slices; t += kRedWaves) s += part[(size_t)t * M + i];
   red[g][lane] = s;
   __syncthreads();
   if (g == 0 && i < M) {
-    float tot = red[0][lane];
+    ACC tot = red[0][lane];
     for (int w = 1; w < kRedWaves; ++w) tot += red[w][lane];
-    out[i] = tot;
+    out[i] = (float)tot;
   }
 }
 
@@ -1183,11 +1184,12 @@ __global__ void finalize_full_kernel(FinalizeArgs a) {
 // N = 100000, D = 32, K = 64: 40.0 -> 36.3 µs; full N = 1500, D = 4, K = 3: 42.6 -> 39.9.
 constexpr int kFusedFinLoads = 4096;
 constexpr int kFusedFinJP = 512, kFusedFinK = 256;
+template <typename ACC>
 __global__ __launch_bounds__(64 * kRedWaves) void reduce_finalize_kernel(FinalizeArgs a, const float* part, int slices,
                                                                          float* stats, LlFold ll) {
-  __shared__ float red[kRedWaves][kFusedFinJP];
+  __shared__ ACC red[kRedWaves][kFusedFinJP];
   __shared__ float row[kFusedFinJP];
-  __shared__ float nkp[kFusedFinK * kRedWaves];
+  __shared__ ACC nkp[kFusedFinK * kRedWaves];
   __shared__ float scratch[32];
   const int b = blockIdx.y, k = blockIdx.x, tid = threadIdx.x, lane = tid & 63, g = tid >> 6;
   const int K = a.K, JP = a.JP;
@@ -1203,7 +1205,7 @@ __global__ __launch_bounds__(64 * kRedWaves) void reduce_finalize_kernel(Finaliz
   const int64_t M = (int64_t)a.B * K * JP;
   const float* prow = part + ((size_t)b * K + k) * JP;
   for (int c = lane; c < JP; c += 64) {
-    float s = 0.f;
+    ACC s = 0;
 #pragma unroll 4
     for (int t = g; t < slices; t += kRedWaves) s += prow[(size_t)t * M + c];
     red[g][c] = s;
@@ -1214,7 +1216,7 @@ __global__ __launch_bounds__(64 * kRedWaves) void reduce_finalize_kernel(Finaliz
   const float* pn = part + (size_t)b * K * JP + a.nk_col;
   for (int e = tid; e < K * kRedWaves; e += blockDim.x) {
     const int k2 = e / kRedWaves, w = e % kRedWaves;
-    float s = 0.f;
+    ACC s = 0;
 #pragma unroll 4
     for (int t = w; t < slices; t += kRedWaves) s += pn[(size_t)t * M + (size_t)k2 * JP];
     nkp[e] = s;
@@ -1222,16 +1224,16 @@ __global__ __launch_bounds__(64 * kRedWaves) void reduce_finalize_kernel(Finaliz
   __syncthreads();
   float wsum = 0.f;
   for (int k2 = tid; k2 < K; k2 += blockDim.x) {
-    float nk = nkp[k2 * kRedWaves];
+    ACC nk = nkp[k2 * kRedWaves];
     for (int w = 1; w < kRedWaves; ++w) nk += nkp[k2 * kRedWaves + w];
-    wsum += clamp_lo(nk / (float)a.N, a.min_weight);
+    wsum += clamp_lo((float)nk / (float)a.N, a.min_weight);
   }
   const float total = block_sum(wsum, scratch);   // (its barriers also cover red)
   for (int c = tid; c < JP; c += blockDim.x) {
-    float tot = red[0][c];
+    ACC tot = red[0][c];
     for (int w = 1; w < kRedWaves; ++w) tot += red[w][c];
-    row[c] = tot;
-    if (stats) stats[((size_t)b * K + k) * JP + c] = tot;
+    row[c] = (float)tot;
+    if (stats) stats[((size_t)b * K + k) * JP + c] = (float)tot;
   }
   __syncthreads();
   if (g == 0) finalize_comp(a, b, k, row, total);
@@ -1448,24 +1450,31 @@ static int reduce_groups(int slices, int64_t M, int64_t tmp_floats) {
 }
 
 // The first stage: `groups` sums of consecutive slices into tmp; returns how many.
+template <typename ACC>
 static int reduce_first(const float* part, int slices, int64_t M, int groups, float* tmp, hipStream_t s) {
   const int per = (slices + groups - 1) / groups;
   groups = (slices + per - 1) / per;  // every group non-empty
-  reduce_slices_kernel<<<dim3((unsigned)((M + 63) / 64), groups), 64 * kRedWaves, 0, s>>>(part, slices, M, tmp, per,
-                                                                                          LlFold{});
+  reduce_slices_kernel<ACC><<<dim3((unsigned)((M + 63) / 64), groups), 64 * kRedWaves, 0, s>>>(part, slices, M, tmp, per,
+                                                                                               LlFold{});
   return groups;
 }
 
-void launch_reduce_slices(const float* part, int slices, int64_t M, float* out, hipStream_t s, float* tmp,
+template <typename ACC>
+static void reduce_slices(const float* part, int slices, int64_t M, float* out, hipStream_t s, float* tmp,
                           int64_t tmp_floats, const LlFold* ll) {
   const int groups = tmp ? reduce_groups(slices, M, tmp_floats) : 1;
   const LlFold lf = ll ? *ll : LlFold{};
   const unsigned last = (unsigned)((M + 63) / 64) + (ll ? 1u : 0u);
   if (groups > 1) {
-    slices = reduce_first(part, slices, M, groups, tmp, s);
+    slices = reduce_first<ACC>(part, slices, M, groups, tmp, s);
     part = tmp;
   }
-  reduce_slices_kernel<<<last, 64 * kRedWaves, 0, s>>>(part, slices, M, out, slices, lf);
+  reduce_slices_kernel<ACC><<<last, 64 * kRedWaves, 0, s>>>(part, slices, M, out, slices, lf);
+}
+
+void launch_reduce_slices(const float* part, int slices, int64_t M, float* out, hipStream_t s, float* tmp,
+                          int64_t tmp_floats, const LlFold* ll, bool wide) {
+  (wide ? reduce_slices<double> : reduce_slices<float>)(part, slices, M, out, s, tmp, tmp_floats, ll);
 }
 
 bool reduce_finalize_fits(const FinalizeArgs& a, int slices, int64_t tmp_floats) {
@@ -1474,18 +1483,24 @@ bool reduce_finalize_fits(const FinalizeArgs& a, int slices, int64_t tmp_floats)
   return !a.skip && a.JP <= kFusedFinJP && (int64_t)a.B * a.K <= kFusedFinK && (int64_t)a.K * (groups > 1 ? groups : slices) <= kFusedFinLoads;
 }
 
-void launch_reduce_finalize(const FinalizeArgs& a, const float* part, int slices, float* tmp, int64_t tmp_floats,
+template <typename ACC>
+static void reduce_finalize(const FinalizeArgs& a, const float* part, int slices, float* tmp, int64_t tmp_floats,
                             const LlFold& ll, hipStream_t s) {
   const int64_t M = (int64_t)a.B * a.K * a.JP;
   const int groups = reduce_groups(slices, M, tmp_floats);
   if (groups > 1) {
-    slices = reduce_first(part, slices, M, groups, tmp, s);
+    slices = reduce_first<ACC>(part, slices, M, groups, tmp, s);
     part = tmp;
   }
   // (tied: its covariance update reads the statistics rows)
-  reduce_finalize_kernel<<<dim3(a.K + 1, a.B), 64 * kRedWaves, 0, s>>>(a, part, slices,
-                                                                      a.cov == TIED ? const_cast<float*>(a.stats) : nullptr, ll);
+  reduce_finalize_kernel<ACC><<<dim3(a.K + 1, a.B), 64 * kRedWaves, 0, s>>>(
+      a, part, slices, a.cov == TIED ? const_cast<float*>(a.stats) : nullptr, ll);
   if (a.cov == TIED) finalize_tied_kernel<<<dim3(a.D, a.B, (a.D + 63) / 64), 64 * kTiedWaves, 0, s>>>(a);
+}
+
+void launch_reduce_finalize(const FinalizeArgs& a, const float* part, int slices, float* tmp, int64_t tmp_floats,
+                            const LlFold& ll, hipStream_t s, bool wide) {
+  (wide ? reduce_finalize<double> : reduce_finalize<float>)(a, part, slices, tmp, tmp_floats, ll, s);
 }
 
 __global__ void take_status_kernel(unsigned* sticky, uint32_t* out) {

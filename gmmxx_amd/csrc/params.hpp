@@ -110,14 +110,16 @@ struct LlFold {
   const unsigned* status;
   unsigned* sticky;
 };
-void launch_reduce_slices(const float* part, int slices, int64_t M, float* out, hipStream_t s,
-                          float* tmp = nullptr, int64_t tmp_floats = 0, const LlFold* ll = nullptr);
+// wide: summed in double (one-block slices: as many partials as row blocks, whose fp32
+// running sum would lose more than the fp32 accumulation within longer slices).
+void launch_reduce_slices(const float* part, int slices, int64_t M, float* out, hipStream_t s, float* tmp = nullptr,
+                          int64_t tmp_floats = 0, const LlFold* ll = nullptr, bool wide = false);
 void launch_finalize(const FinalizeArgs& a, hipStream_t s);
 // Slice reduction, log-likelihood (its status words unused) and finalize with the
 // last reduction and the finalize in one launch, for statistics small enough.
 bool reduce_finalize_fits(const FinalizeArgs& a, int slices, int64_t tmp_floats);
 void launch_reduce_finalize(const FinalizeArgs& a, const float* part, int slices, float* tmp, int64_t tmp_floats,
-                            const LlFold& ll, hipStream_t s);
+                            const LlFold& ll, hipStream_t s, bool wide);
 void launch_unpack(const UnpackArgs& a, int B, hipStream_t s);
 void launch_pack(const PackArgs& a, int B, hipStream_t s);
 void launch_gram(const float* x, int B, int64_t N, int D, int slices, int64_t rows_per_slice, float* part,
