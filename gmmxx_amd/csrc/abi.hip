@@ -255,7 +255,7 @@ int plan_problem(const gmmxx_problem* p, Plan* pl) {
   q.chol_m = (q.cov == TIED) ? q.B : (q.cov == FULL ? q.B * q.K : 0);
   if (q.fw) {
     // E-step: one wave per 32-row block.  Statistics: eight-wave workgroups of 16
-    // components over row slices, one per CU (em_full_stats.hip), or, for few
+    // components over row slices (em_full_stats.hip), or, for few
     // components, workgroups of four waves (four components; at D = 128 two
     // components of two waves), as many as one round of resident waves: 8, 4 and 2 waves per SIMD at
     // DP = 32, 64 and 128 (the kernels' register counts), so 2048, 1024 and 512
@@ -264,8 +264,16 @@ int plan_problem(const gmmxx_problem* p, Plan* pl) {
     q.fw_tile = fw_stats_tile_pays(q.D, q.DP, q.K);
     const int64_t groups =
         (q.fw_tile ? fw_stats_tile_groups(q.D, q.K) : (q.DP == 128 ? (q.K + 1) / 2 : (q.K + 3) / 4)) * (int64_t)q.B;
-    const int64_t target = q.fw_tile ? 256 : (q.DP == 32 ? 2048 : (q.DP == 64 ? 1024 : 512));
+    const int64_t target =
+        q.fw_tile ? (q.D <= 32 && q.K <= 16 ? 512 : 256) : (q.DP == 32 ? 2048 : (q.DP == 64 ? 1024 : 512));
     int64_t fs = std::max<int64_t>(1, (target + groups - 1) / groups);
+    // (16-component kernel: two rounds of shorter slices where one round's pass 2048 rows,
+    // and from the start where they cost nothing (one component tile at D <= 32), since long
+    // fp32 sums lose bits.  N = 250000, D = 17, K = 16: Σ r x xᵀ 1.16e-7 off with 256 slices, 0.7e-7
+    // with 512, 0.85e-7 with fw_stats_kernel's 512; N = 250000, D = 128, K = 12: Σ r x xᵀ 5.2e-7 off with
+    // 64 slices, 2.5e-7 with 128, 3.8e-7 with fw_stats128_kernel's 85; 1.18 -> 1.17 ms.  Two
+    // rounds of slices of 1000 rows took up to 7 % longer.)
+    if (q.fw_tile && q.N > 2048 * fs) fs *= 2;
     fs = std::min(fs, std::max<int64_t>(1, row_blocks / kMinBlocksPerSlice));
     q.fw_rows = ((q.N + fs - 1) / fs + kBN - 1) / kBN * kBN;
     q.fw_slices = (int)((q.N + q.fw_rows - 1) / q.fw_rows);
@@ -464,8 +472,11 @@ LlFold ll_fold(const Plan& pl, void* ws, int parts, double inv_total, float* out
 int stat_slices(const Plan& pl) {
   return pl.fw ? pl.fw_slices : (pl.fused ? pl.fparts : (pl.coop ? pl.cspb : (pl.xch ? pl.xslices : pl.slices)));
 }
-// Whether the partial sums are those of one-block slices (the tile pass's own).
-bool wide_sums(const Plan& pl) { return pl.short_slices && !(pl.fw || pl.fused || pl.coop || pl.xch); }
+// Whether the slice sums are added in double: one-block slices (the tile pass's own), and
+// the 16-component statistics, whose slices are fewer and longer than fw_stats128_kernel's.
+bool wide_sums(const Plan& pl) {
+  return pl.fw ? pl.fw_tile : pl.short_slices && !(pl.fused || pl.coop || pl.xch);
+}
 // The tile-partial buffer is free once the statistics are being reduced: it is
 // the scratch of the grouped slice reduction.
 float* red_tmp(const Plan& pl, void* ws) { return at<float>(ws, pl.o_pms); }
@@ -492,6 +503,8 @@ FwArgs fw_args(const Plan& pl, const void* x, void* ws) {
   a.cconst = at<float4>(ws, pl.o_cconst);
   a.l2 = at<float>(ws, pl.o_l2w);
   a.lse2 = at<float>(ws, pl.o_lse2);
+  // (the tile partials' buffer, unused here until the slice reduction: 8 bytes per row)
+  a.lse_lo = pl.fw_tile ? at<float>(ws, pl.o_pms) : nullptr;
   a.ll_part = at<double>(ws, pl.o_ll);
   a.part_stats = at<float>(ws, pl.o_pstats);
   a.JP = pl.JP;
@@ -963,7 +976,7 @@ int gmmxx_hip_estep_stats(const gmmxx_problem* p, const void* x, const float* me
     if ((rc = run_fw(pl, 0, a, s)) || (rc = run_fw(pl, 1, a, s))) return rc;
     const LlFold ll = ll_fold(pl, ws, ll_parts(pl), 1.0, ll_sum);
     launch_reduce_slices(at<float>(ws, pl.o_pstats), stat_slices(pl), (int64_t)pl.B * pl.K * pl.JP,
-                         at<float>(ws, pl.o_stats), s, red_tmp(pl, ws), red_tmp_floats(pl), &ll);
+                         at<float>(ws, pl.o_stats), s, red_tmp(pl, ws), red_tmp_floats(pl), &ll, wide_sums(pl));
     if ((rc = check_hip("full-covariance statistics reduction"))) return rc;
   } else if (pl.fused || pl.coop || pl.single || pl.xch) {
     if (pl.coop) {
@@ -1046,13 +1059,14 @@ int gmmxx_hip_estep_stats_topk(const gmmxx_problem* p, const void* x, const floa
     if ((rc = run_fw(pl, 0, a, s)) || (rc = run_fw(pl, 1, a, s))) return rc;
     const LlFold ll = ll_fold(pl, ws, ll_parts(pl), 1.0, ll_sum);
     launch_reduce_slices(at<float>(ws, pl.o_pstats), stat_slices(pl), (int64_t)pl.B * pl.K * pl.JP,
-                         at<float>(ws, pl.o_stats), s, red_tmp(pl, ws), red_tmp_floats(pl), &ll);
+                         at<float>(ws, pl.o_stats), s, red_tmp(pl, ws), red_tmp_floats(pl), &ll, wide_sums(pl));
   } else if (pl.fw) {
     // the E-step's (B, K, N) log2 logits, transposed to (B, N, K) for the per-row
     // top-k selection (threshold, index, top-k log-normaliser), then the statistics
     // over each row's kept components
     FwArgs a = fw_args(pl, x, ws);
     a.ll_part = nullptr;
+    a.lse_lo = nullptr;      // (lse2 becomes the top-k log-normaliser)
     if ((rc = run_fw(pl, 0, a, s))) return rc;
     float* logits = at<float>(ws, tl.o_logits);
     launch_fw_proba(a.l2, a.lse2, logits, pl.B, pl.N, pl.K, s, /*raw=*/true);
@@ -1063,7 +1077,7 @@ int gmmxx_hip_estep_stats_topk(const gmmxx_problem* p, const void* x, const floa
     a.thr_idx = thri;
     if ((rc = run_fw(pl, 1, a, s))) return rc;
     launch_reduce_slices(at<float>(ws, pl.o_pstats), stat_slices(pl), (int64_t)pl.B * pl.K * pl.JP,
-                         at<float>(ws, pl.o_stats), s, red_tmp(pl, ws), red_tmp_floats(pl));
+                         at<float>(ws, pl.o_stats), s, red_tmp(pl, ws), red_tmp_floats(pl), nullptr, wide_sums(pl));
     launch_ll_reduce(tll, pl.B * sel_blocks, 1.0, ll_sum, s);
   } else if (top_k == 1) {
     // Hard assignment: the first-argmax pass gives each row's maximum (the

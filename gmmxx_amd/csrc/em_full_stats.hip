@@ -16,7 +16,9 @@
 // the same number of tiles), so the waves' MFMA counts are equal.  Rows pass
 // through LDS in blocks of 32, twice buffered, one barrier per block: transposed
 // fp32 columns (the x_i broadcast) and their three bf16 parts (the B operand),
-// staged with the responsibilities 2^(l2 - lse2), one per thread.
+// staged with the responsibilities 2^(l2 - lse2), one per thread (lse2 with the remainder of
+// its last rounding: of a row that one component dominates the others' share is below half
+// a unit of lse2, and without it every such r is too large, N_k by up to 3e-7).
 //
 // Bound by MFMA and VALU issue, which overlap in part (per wave and block at D = 64:
 // 126 MFMAs, 2016 cycles, beside about 370 VALU instructions; 0.117 ms of MFMA at
@@ -95,7 +97,7 @@ __device__ __forceinline__ void stats_part(const FwArgs& a, int ctile, StatsLds<
   const bf16x2 nlo = __builtin_bit_cast(bf16x2, clo), nhi = __builtin_bit_cast(bf16x2, chi);
 
   // ---- loader: raw values of a block, then (one block later) its staged form ----
-  float px[UP][4], pl[CT], pn = 0.f;
+  float px[UP][4], pl[CT], pn = 0.f, pn_lo = 0.f;
   auto fetch = [&](int64_t n0) {
     const int left = r1 - n0 < kBN ? (int)(r1 - n0) : kBN;
     const float* blk = xb + (size_t)n0 * D;
@@ -110,6 +112,7 @@ __device__ __forceinline__ void stats_part(const FwArgs& a, int ctile, StatsLds<
     }
     const int64_t n = n0 + (rr < left ? rr : left - 1);
     pn = lse2[n];
+    if (a.lse_lo) pn_lo = a.lse_lo[(size_t)b * N + n];
     if (!a.hard) {
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct) {
@@ -145,7 +148,7 @@ __device__ __forceinline__ void stats_part(const FwArgs& a, int ctile, StatsLds<
       if (a.hard) {
         r = a.hard_idx[(size_t)b * N + n] == k ? 1.f : 0.f;
       } else {
-        r = fast_exp2(pl[ct] - pn);
+        r = fast_exp2((pl[ct] - pn) - pn_lo);
         if (a.thr2) {      // top-k mode: only the row's kept components
           const float t = a.thr2[(size_t)b * N + n];
           if (!(pl[ct] > t || (pl[ct] == t && k <= a.thr_idx[(size_t)b * N + n]))) r = 0.f;

@@ -280,10 +280,14 @@ __global__ __launch_bounds__(64 * kFwWaves) void fw_estep_kernel(FwArgs a) {
     }
     if (a.l2 && h == 0 && valid) a.l2[bk * N + n] = l2;
   }
-  const float lse = a.hard ? best : m + __log2f(s);
+  const float lg = __log2f(s), lse = a.hard ? best : m + lg;
   double ll = 0.0;
   if (h == 0 && valid) {
     a.lse2[(size_t)b * N + n] = lse;
+    if (a.lse_lo) {          // (two-sum: lse + the remainder = m + lg)
+      const float t = lse - m;
+      a.lse_lo[(size_t)b * N + n] = (m - (lse - t)) + (lg - t);
+    }
     if (a.hard) a.hard_idx[(size_t)b * N + n] = bidx;
     if (a.scores) a.scores[(size_t)b * N + n] = lse * kLn2;
     if (a.labels) a.labels[(size_t)b * N + n] = bidx;

@@ -128,6 +128,7 @@ struct FwArgs {
   const float4* cconst;
   float* l2;                   // [B][K][N] log2 logits (E-step output, statistics input), or null
   float* lse2;                 // [B][N] log2 row log-normalisers
+  float* lse_lo;               // [B][N] what lse2 lost in its last rounding, or null (16-component statistics)
   float* scores;               // [B][N] natural-log scores, or null
   int64_t* labels;             // [B][N] first argmax, or null
   double* ll_part;             // [B][fw_eblocks(N)] natural-log partial sums, or null
