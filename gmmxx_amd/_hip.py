@@ -359,8 +359,8 @@ def em_step_noalloc(covariance_type: str, x: torch.Tensor, means: torch.Tensor, 
                     weights: torch.Tensor, lower_bound_out: torch.Tensor, *, reg_covar: float = 1e-6,
                     min_weight: float = 1e-8, gram_xx: Optional[torch.Tensor] = None) -> None:
     """em_step on the library's static device scratch (gmmxx_hip_em_step_noalloc):
-    no workspace is allocated; problems needing more than 64 MiB of workspace
-    are refused.  Calls on one device share the scratch and must not overlap."""
+    no workspace is allocated; problems needing more than 64 MiB, with the leanest
+    kernels too, are refused.  Calls on one device share the scratch and must not overlap."""
     require_hip()
     x = _device_tensor(x, "x")
     B, N, D, K = _shape(x, means)

@@ -92,7 +92,9 @@ int dp_for(int64_t d) {
   return -1;
 }
 
-int plan_problem(const gmmxx_problem* p, Plan* pl) {
+// lean: the plan of an EM iteration with less scratch (gmmxx_hip_em_step_noalloc): the
+// kernels with smaller partial statistics, two passes for spherical bf16.
+int plan_problem(const gmmxx_problem* p, Plan* pl, bool lean = false) {
   if (!p) return fail(GMMXX_ERR_INVALID_ARGUMENT, "problem descriptor is NULL");
   if (p->covariance_type < 0 || p->covariance_type > 3)
     return fail(GMMXX_ERR_INVALID_ARGUMENT, "covariance_type must be 0..3");
@@ -193,7 +195,8 @@ int plan_problem(const gmmxx_problem* p, Plan* pl) {
   // whole groups (multiples of 8 groups keep each group on one XCD).
   // GMMXX_HIP_NO_COOP=1 selects the two-pass kernels instead.
   const char* no_coop = getenv("GMMXX_HIP_NO_COOP");
-  q.coop = sph_bf && !q.fused && q.K <= kCoopComps * kMaxCoopGroup && !(no_coop && no_coop[0] == '1');
+  q.coop = sph_bf && !q.fused && q.K <= kCoopComps * kMaxCoopGroup && !(no_coop && no_coop[0] == '1') &&
+           (!lean || (q.D == 128 && q.K > kCoopComps));
   if (q.coop) {
     q.cDP = round_up(std::max(q.D, 1), 32);
     q.cG = (q.K + kCoopComps - 1) / kCoopComps;
@@ -261,7 +264,7 @@ int plan_problem(const gmmxx_problem* p, Plan* pl) {
     // DP = 32, 64 and 128 (the kernels' register counts), so 2048, 1024 and 512
     // workgroups (at D = 64, 2048 measured 5 % slower per EM iteration).
     q.fw_eblk = fw_eblocks(q.N);
-    q.fw_tile = fw_stats_tile_pays(q.D, q.DP, q.K);
+    q.fw_tile = !lean && fw_stats_tile_pays(q.D, q.DP, q.K);
     const int64_t groups =
         (q.fw_tile ? fw_stats_tile_groups(q.D, q.K) : (q.DP == 128 ? (q.K + 1) / 2 : (q.K + 3) / 4)) * (int64_t)q.B;
     const int64_t target =
@@ -291,7 +294,7 @@ int plan_problem(const gmmxx_problem* p, Plan* pl) {
   q.o_waug = take(sph_bf ? BK * 32 * 2 : 0);
   // The bf16 means, their factor and the augmented constants of s·(x·μ - ‖x‖²/2 + C'):
   // the single passes and the label pass.
-  q.sb = sph_bf && q.K <= kCoopComps * kMaxCoopGroup;
+  q.sb = sph_bf && (lean ? q.coop || q.fused : q.K <= kCoopComps * kMaxCoopGroup);
   q.o_wmu = take(q.sb ? BK * q.DP * 2 : 0);
   q.o_wsc = take(q.sb ? BK * 4 : 0);
   q.o_waugs = take(q.sb ? BK * 16 * 2 : 0);
@@ -836,12 +839,9 @@ int gmmxx_hip_workspace_init(const gmmxx_problem* p, void* ws, int64_t ws_bytes,
   return check_hip("workspace_init");
 }
 
-int gmmxx_hip_em_phase(const gmmxx_problem* p, int phase, const void* x, float* means, float* covs,
-                       float* weights, const float* gram, double reg_covar, double min_weight,
-                       float* lower_bound, void* ws, int64_t ws_bytes, void* stream) {
-  Plan pl;
-  int rc = begin(p, &pl, x, ws, ws_bytes);
-  if (rc) return rc;
+static int em_phase(const Plan& pl, int phase, const void* x, float* means, float* covs, float* weights,
+                    const float* gram, double reg_covar, double min_weight, float* lower_bound, void* ws,
+                    void* stream) {
   if (!means || !covs || !weights || !lower_bound) return fail(GMMXX_ERR_INVALID_ARGUMENT, "NULL parameter buffer");
   if (pl.cov == TIED && !gram) return fail(GMMXX_ERR_INVALID_ARGUMENT, "tied EM needs the XᵀX buffer");
   if (!(min_weight > 0.0)) return fail(GMMXX_ERR_INVALID_ARGUMENT, "min_weight must be positive");
@@ -912,22 +912,25 @@ int gmmxx_hip_em_phase(const gmmxx_problem* p, int phase, const void* x, float* 
   }
 }
 
-int gmmxx_hip_em_step(const gmmxx_problem* p, const void* x, float* means, float* covs, float* weights,
-                      const float* gram, double reg_covar, double min_weight, float* lower_bound,
-                      void* ws, int64_t ws_bytes, void* stream) {
-  int last = GMMXX_PHASE_FINALIZE;
-  // A single pass with small statistics: the reduction and the finalize share a launch.
+int gmmxx_hip_em_phase(const gmmxx_problem* p, int phase, const void* x, float* means, float* covs,
+                       float* weights, const float* gram, double reg_covar, double min_weight,
+                       float* lower_bound, void* ws, int64_t ws_bytes, void* stream) {
   Plan pl;
-  int prc = plan_problem(p, &pl);
-  if (prc) return prc;
+  const int rc = begin(p, &pl, x, ws, ws_bytes);
+  if (rc) return rc;
+  return em_phase(pl, phase, x, means, covs, weights, gram, reg_covar, min_weight, lower_bound, ws, stream);
+}
+
+static int em_step(const Plan& pl, const void* x, float* means, float* covs, float* weights, const float* gram,
+                   double reg_covar, double min_weight, float* lower_bound, void* ws, void* stream) {
+  // A single pass with small statistics: the reduction and the finalize share a launch.
   FinalizeArgs f{};
-  const bool fuse = ll_in_pass(pl) && !(pl.coop && pl.cG > 1) && !pl.xch && ws && (f = finalize_args(
+  const bool fuse = ll_in_pass(pl) && !(pl.coop && pl.cG > 1) && !pl.xch && (f = finalize_args(
       pl, ws, gram, reg_covar, min_weight, pl.N, means, covs, weights, nullptr),
       reduce_finalize_fits(f, stat_slices(pl), red_tmp_floats(pl)));
-  if (fuse) last = GMMXX_PHASE_STATS_TILE;
+  const int last = fuse ? GMMXX_PHASE_STATS_TILE : GMMXX_PHASE_FINALIZE;
   for (int ph = GMMXX_PHASE_PREPARE; ph <= last; ++ph) {
-    const int rc = gmmxx_hip_em_phase(p, ph, x, means, covs, weights, gram, reg_covar, min_weight,
-                                      lower_bound, ws, ws_bytes, stream);
+    const int rc = em_phase(pl, ph, x, means, covs, weights, gram, reg_covar, min_weight, lower_bound, ws, stream);
     if (rc) return rc;
   }
   if (!fuse) return GMMXX_OK;
@@ -939,12 +942,28 @@ int gmmxx_hip_em_step(const gmmxx_problem* p, const void* x, float* means, float
   return check_hip("reduction and finalize");
 }
 
+int gmmxx_hip_em_step(const gmmxx_problem* p, const void* x, float* means, float* covs, float* weights,
+                      const float* gram, double reg_covar, double min_weight, float* lower_bound,
+                      void* ws, int64_t ws_bytes, void* stream) {
+  Plan pl;
+  const int rc = begin(p, &pl, x, ws, ws_bytes);
+  if (rc) return rc;
+  return em_step(pl, x, means, covs, weights, gram, reg_covar, min_weight, lower_bound, ws, stream);
+}
+
 int gmmxx_hip_em_step_noalloc(const gmmxx_problem* p, const void* x, float* means, float* covs, float* weights,
                               const float* gram, double reg_covar, double min_weight, float* lower_bound,
                               void* stream) {
   Plan pl;
   int rc = plan_problem(p, &pl);
   if (rc) return rc;
+  if (!x) return fail(GMMXX_ERR_INVALID_ARGUMENT, "x is NULL");
+  // A problem whose faster plan does not fit takes the lean one (spherical bf16
+  // 1594715 x 88, K = 47: 78.7 MB, lean 58.1).
+  if ((int64_t)pl.total > kScratchBytes) {
+    pl = Plan{};
+    if ((rc = plan_problem(p, &pl, /*lean=*/true))) return rc;
+  }
   if ((int64_t)pl.total > kScratchBytes)
     return fail(GMMXX_ERR_WORKSPACE, "problem needs " + std::to_string(pl.total) +
                                          " bytes of scratch, above the no-allocation limit of " +
@@ -955,8 +974,7 @@ int gmmxx_hip_em_step_noalloc(const gmmxx_problem* p, const void* x, float* mean
   // (the coop launcher zeroes its exchange words itself): clear them with a
   // kernel, which a caller may also capture in a graph.
   launch_zero_words(at<unsigned>(ws, pl.o_flags), 2, (hipStream_t)stream);
-  return gmmxx_hip_em_step(p, x, means, covs, weights, gram, reg_covar, min_weight, lower_bound, ws, kScratchBytes,
-                           stream);
+  return em_step(pl, x, means, covs, weights, gram, reg_covar, min_weight, lower_bound, ws, stream);
 }
 
 int gmmxx_hip_estep_stats(const gmmxx_problem* p, const void* x, const float* means, const float* covs,

@@ -143,8 +143,10 @@ int gmmxx_hip_workspace_init(const gmmxx_problem* p, void* workspace, int64_t wo
 /* gmmxx_hip_em_step without a caller workspace: the same kernels run on a
  * static device scratch array of the library (64 MiB per device, held for
  * the life of the process), so the call allocates nothing and takes no
- * workspace arguments.  Problems whose gmmxx_hip_workspace_bytes exceeds
- * 64 MiB are refused with GMMXX_ERR_WORKSPACE before any launch.  Every call
+ * workspace arguments.  Where gmmxx_hip_workspace_bytes exceeds 64 MiB, kernels with
+ * smaller partial statistics run instead (same results to the tolerances of the covariance
+ * type); problems too large for those too are refused with GMMXX_ERR_WORKSPACE
+ * before any launch.  Every call
  * on one device shares that device's scratch: calls that overlap on one
  * device (two streams, two threads) race and must be ordered by the caller.
  * The call clears the scratch's status words first and there is no workspace
