@@ -93,7 +93,7 @@ int dp_for(int64_t d) {
 }
 
 // lean: the plan of an EM iteration with less scratch (gmmxx_hip_em_step_noalloc): the
-// kernels with smaller partial statistics, two passes for spherical bf16.
+// kernels with smaller partial statistics, two passes for spherical bf16, no one-block slices.
 int plan_problem(const gmmxx_problem* p, Plan* pl, bool lean = false) {
   if (!p) return fail(GMMXX_ERR_INVALID_ARGUMENT, "problem descriptor is NULL");
   if (p->covariance_type < 0 || p->covariance_type > 3)
@@ -167,7 +167,7 @@ int plan_problem(const gmmxx_problem* p, Plan* pl, bool lean = false) {
   // Problems that leave most CUs idle: one block per slice, the shortest chain.  Their sums
   // are added in double: in fp32 the statistics of 800 rows were 1.2 to 1.9 times as far
   // from float64 as with three blocks per slice.
-  q.short_slices = row_blocks * q.ktiles * q.B <= 256;
+  q.short_slices = !lean && row_blocks * q.ktiles * q.B <= 256;
   slices = std::min(slices, std::max<int64_t>(1, row_blocks / (q.short_slices ? 1 : kMinBlocksPerSlice)));
   q.rows_per_slice = ((q.N + slices - 1) / slices + kBN - 1) / kBN * kBN;
   q.slices = (int)((q.N + q.rows_per_slice - 1) / q.rows_per_slice);
