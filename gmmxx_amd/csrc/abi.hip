@@ -264,19 +264,26 @@ int plan_problem(const gmmxx_problem* p, Plan* pl, bool lean = false) {
     // DP = 32, 64 and 128 (the kernels' register counts), so 2048, 1024 and 512
     // workgroups (at D = 64, 2048 measured 5 % slower per EM iteration).
     q.fw_eblk = fw_eblocks(q.N);
-    q.fw_tile = !lean && fw_stats_tile_pays(q.D, q.DP, q.K);
-    const int64_t groups =
-        (q.fw_tile ? fw_stats_tile_groups(q.D, q.K) : (q.DP == 128 ? (q.K + 1) / 2 : (q.K + 3) / 4)) * (int64_t)q.B;
-    const int64_t target =
-        q.fw_tile ? (q.D <= 32 && q.K <= 16 ? 512 : 256) : (q.DP == 32 ? 2048 : (q.DP == 64 ? 1024 : 512));
-    int64_t fs = std::max<int64_t>(1, (target + groups - 1) / groups);
-    // (16-component kernel: two rounds of shorter slices where one round's pass 2048 rows,
-    // and from the start where they cost nothing (one component tile at D <= 32), since long
-    // fp32 sums lose bits.  N = 250000, D = 17, K = 16: Σ r x xᵀ 1.16e-7 off with 256 slices, 0.7e-7
-    // with 512, 0.85e-7 with fw_stats_kernel's 512; N = 250000, D = 128, K = 12: Σ r x xᵀ 5.2e-7 off with
-    // 64 slices, 2.5e-7 with 128, 3.8e-7 with fw_stats128_kernel's 85; 1.18 -> 1.17 ms.  Two
-    // rounds of slices of 1000 rows took up to 7 % longer.)
-    if (q.fw_tile && q.N > 2048 * fs) fs *= 2;
+    // Up to K = 8 the tile of 16 is mostly padding: N = 262144, D = 64, K = 8 0.137 ms against
+    // 0.115 of the per-component kernels.  Above, whole calls (E-step included):
+    // D = 64, K = 9 0.277 against 0.309, K = 17 0.446 / 0.473; D = 32, K = 17 0.187 / 0.204, K = 33
+    // 0.318 / 0.349; N = 130000, D = 128, K = 9 0.698 / 0.723, K = 17 1.00 / 1.09.
+    q.fw_tile = !lean && q.K > 8;
+    auto one_round = [&](int64_t target, int64_t groups) {
+      return std::max<int64_t>(1, (target + groups * q.B - 1) / (groups * q.B));
+    };
+    int64_t fs = one_round(q.DP == 32 ? 2048 : (q.DP == 64 ? 1024 : 512), q.DP == 128 ? (q.K + 1) / 2 : (q.K + 3) / 4);
+    if (q.fw_tile) {
+      // Long fp32 sums lose bits: two rounds where slices would pass 2048 rows, or 1024 and
+      // the per-component kernels' length, and where it costs nothing (one component tile
+      // at D <= 32).  Σ r x xᵀ against float64: N = 250000, D = 128, K = 12 5.2e-7
+      // with 64 slices, 2.5e-7 with 128, 3.8e-7 with the other kernels' 86 (1.18 -> 1.17 ms);
+      // D = 17, K = 16 1.16e-7 with 256, 0.7e-7 with 512 (0.149 -> 0.150).  Two rounds of shorter
+      // slices took up to 7 % longer.
+      int64_t ts = one_round(q.D <= 32 && q.K <= 16 ? 512 : 256, fw_stats_tile_groups(q.D, q.K));
+      if (q.N > 2048 * ts || (ts < fs && q.N > 1024 * ts)) ts *= 2;
+      fs = ts;
+    }
     fs = std::min(fs, std::max<int64_t>(1, row_blocks / kMinBlocksPerSlice));
     q.fw_rows = ((q.N + fs - 1) / fs + kBN - 1) / kBN * kBN;
     q.fw_slices = (int)((q.N + q.fw_rows - 1) / q.fw_rows);

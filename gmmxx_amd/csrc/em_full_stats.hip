@@ -24,9 +24,8 @@
 // 126 MFMAs, 2016 cycles, beside about 370 VALU instructions; 0.117 ms of MFMA at
 // N = 262144, K = 32).  Statistics launch, fw_stats_kernel -> here: D = 64, K = 32
 // 0.390 -> 0.254 ms; D = 32, K = 32 0.181 -> 0.112; D = 33, K = 32 0.38 -> 0.164;
-// N = 130000: D = 128, K = 16 0.389 -> 0.237; D = 80, K = 24 0.80 -> 0.27.  The error
-// of the sums against float64 is the same (2e-7).
-//
+// N = 130000: D = 128, K = 16 0.389 -> 0.237; D = 80, K = 24 0.80 -> 0.27.  Error of
+// Σ r x xᵀ against float64 at N = 262144, D = 64, K = 32: 2.6e-7 -> 1.9e-7.
 //
 // 16x16x32 bf16 MFMA operand layout: lane l supplies A[i = l % 16][k = 8 (l / 16) .. +7]
 // and B[k = 8 (l / 16) .. +7][j = l % 16]; accumulator register v of lane l holds
@@ -316,17 +315,6 @@ void launch_tile(const FwArgs& a, int slices, hipStream_t s) {
 int fw_stats_tile_groups(int D, int K) {
   const int per = 16 * comp_tiles(D, K);
   return (K + per - 1) / per * parts_of(D);
-}
-
-// Measured against fw_stats_kernel / fw_stats128_kernel: 0.62 of their time per
-// component where both compute the same columns (D = 32, 64, 128), the components
-// padded to whole tiles of 16 and the columns to 16 instead of 32, 64 or 128.
-// N = 262144, D = 64: K = 8 0.137 against 0.115 ms, K = 9 0.134 / 0.159, K = 16
-// 0.143 / 0.207, K = 17 0.243 / 0.259, K = 32 0.254 / 0.390.  Up to K = 8 the other
-// kernels' shorter slices also sum fewer rows in fp32.
-bool fw_stats_tile_pays(int D, int DP, int K) {
-  const int64_t nj = (D + 15) / 16, dj = DP / 16, per = 16 * comp_tiles(D, K), slots = (K + per - 1) / per * per;
-  return K > 8 && 62 * nj * (nj + 1) * slots < 100 * dj * (dj + 1) * (int64_t)K;
 }
 
 int launch_fw_stats_tile(const FwArgs& a, int slices, hipStream_t s) {

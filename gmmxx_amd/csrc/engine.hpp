@@ -156,7 +156,6 @@ int launch_fw(int dp, int phase, const FwArgs& a, int slices, hipStream_t s);
 // The statistics by 16-component workgroups (em_full_stats.hip) over slices x
 // fw_stats_tile_groups(D, K) x B; 16 < D <= 128.
 int fw_stats_tile_groups(int D, int K);
-bool fw_stats_tile_pays(int D, int DP, int K);
 int launch_fw_stats_tile(const FwArgs& a, int slices, hipStream_t s);
 // proba[b][n][k] = 2^(l2[b][k][n] - lse2[b][n]), or (raw) the log2 logits l2 themselves, transposed.
 void launch_fw_proba(const float* l2, const float* lse2, float* proba, int B, int64_t N, int K, hipStream_t s,

@@ -1,6 +1,6 @@
-"""The 16-component statistics kernel of full covariance at D > 16: its column groups
-(every multiple of 16 up to 128 and one more), component tiles, short slices, and the
-hard and top-k responsibilities, against the oracle.
+"""The 16-component statistics kernel of full covariance at D > 16 (every K > 8): its
+column groups (every multiple of 16 up to 128 and one more), component tiles (two at
+D <= 32, K > 16), short slices, and the hard and top-k responsibilities, against the oracle.
 
 Tolerance: fp32 statistics 1e-4 of the statistic's scale, as test_hip_parity; the
 top-k sums likewise (seeded problems without ties at the boundary).
@@ -20,7 +20,7 @@ def _close(got, exp, tol=1e-4):
 
 
 @pytest.mark.parametrize("d,k", [(17, 9), (17, 33), (32, 12), (32, 17), (33, 16), (48, 9), (49, 31), (64, 9), (64, 32),
-                                 (65, 16), (80, 12), (81, 9), (96, 16), (97, 9), (112, 16), (113, 9), (128, 16)])
+                                 (65, 16), (80, 12), (81, 9), (96, 16), (97, 9), (112, 16), (113, 9), (128, 16), (17, 16), (24, 32), (32, 60), (128, 17)])
 @pytest.mark.parametrize("b,n", [(1, 1), (2, 33), (1, 700)])
 def test_statistics_match_oracle(hip, d, k, b, n):
     print(f"[full stats] B={b} N={n} D={d} K={k}", flush=True)
