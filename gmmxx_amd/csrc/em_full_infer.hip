@@ -9,7 +9,10 @@
 //
 // Two components make one 32 x 32 output tile of v_mfma_f32_32x32x16_bf16 (16
 // dims of each x 32 rows), accumulated from -L⁻¹μ by the six products of the split
-// operands down to 2^-24 (L_l x_h, L_m x_m, L_h x_l, L_m x_h, L_h x_m, L_h x_h).
+// operands down to 2^-24, L_h x_h first: it cancels -L⁻¹μ, and the others (L_h x_m,
+// L_h x_l, L_m x_h, L_m x_m, L_l x_h) are rounded at the size of y (smallest first the scores
+// of data 300 from the origin were 2.5 times as far from float64; responsibilities of
+// 16 x 262144 rows, K = 32 382 -> 386 us).
 // Lane l holds 8 of the 16 dims of both components for row l % 32: one swap of the
 // two partial norms between lanes l and l ^ 32 and one addition leave lane half h
 // with the whole norm of its own component.  The pair of step j is (j, KH + j), KH =
@@ -216,17 +219,17 @@ __global__ __launch_bounds__(64 * kWaves, groups_per_cu(KH)) void full16_infer_k
       const float cst = cl[j];
       f32x16 t[kRB];
 #pragma unroll
-      for (int rb = 0; rb < kRB; ++rb) t[rb] = mfma32(Ll, xh[rb], c);
+      for (int rb = 0; rb < kRB; ++rb) t[rb] = mfma32(Lh, xh[rb], c);
 #pragma unroll
-      for (int rb = 0; rb < kRB; ++rb) t[rb] = mfma32(Lm, xm[rb], t[rb]);
+      for (int rb = 0; rb < kRB; ++rb) t[rb] = mfma32(Lh, xm[rb], t[rb]);
 #pragma unroll
       for (int rb = 0; rb < kRB; ++rb) t[rb] = mfma32(Lh, xl[rb], t[rb]);
 #pragma unroll
       for (int rb = 0; rb < kRB; ++rb) t[rb] = mfma32(Lm, xh[rb], t[rb]);
 #pragma unroll
-      for (int rb = 0; rb < kRB; ++rb) t[rb] = mfma32(Lh, xm[rb], t[rb]);
+      for (int rb = 0; rb < kRB; ++rb) t[rb] = mfma32(Lm, xm[rb], t[rb]);
 #pragma unroll
-      for (int rb = 0; rb < kRB; ++rb) t[rb] = mfma32(Lh, xh[rb], t[rb]);
+      for (int rb = 0; rb < kRB; ++rb) t[rb] = mfma32(Ll, xh[rb], t[rb]);
 #pragma unroll
       for (int rb = 0; rb < kRB; ++rb) {
         float q0 = t[rb][0] * t[rb][0], q1 = t[rb][8] * t[rb][8];
