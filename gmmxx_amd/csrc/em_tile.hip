@@ -384,8 +384,10 @@ __global__ __launch_bounds__(512) void em_tile_kernel(TileArgs a) {
   // masks and shifts of `settle` would sit in a loop bound by VALU issue (ten iterations,
   // settled -> by element: spherical 200k x 6, K = 400 2023 -> 1924 us; 400k x 21, K = 705
   // 5858 -> 5573; diag 200k x 6, K = 400 2047 -> 1952; tied 200k x 9, K = 900 4070 -> 3833; at
-  // DP = 64 settled is the faster form: spherical 200k x 50, K = 600 3736 against 3796).
-  constexpr bool BYELEM = XCH && DP <= 32;
+  // DP = 64 settled is the faster form: spherical 200k x 50, K = 600 3736 against 3796), and so
+  // does full covariance at D < 16, where the loads wait beside the features' products (one
+  // iteration, 2 x 1326498 x 14, K = 60 734 -> 704 us; 103 x 2290 x 1, K = 33 159 -> 155).
+  constexpr bool BYELEM = (XCH && DP <= 32) || (COV == FULL && !EX);
   auto rows_left = [&](int64_t n0) -> int { return rend - n0 < kBN ? (int)(rend - n0) : kBN; };
   auto load_chunk = [&](int c, int64_t n0, int left) -> uint4 {
     const int r = c / CPR, cc = (c % CPR) * VEC;
