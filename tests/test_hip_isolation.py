@@ -14,11 +14,14 @@ pytestmark = pytest.mark.gpu
 BF = torch.bfloat16
 
 # (B, N, D, K): one workgroup per problem of two, four and eight waves (1024, 512 and 256
-# workgroups), three row blocks (the staging's buffer count)
-ONE = [(1100, 96, 72, 50), (600, 96, 121, 60), (600, 96, 72, 100), (300, 96, 72, 200), (300, 96, 128, 256)]
+# workgroups), three row blocks (the staging's buffer count); the last in several items per
+# problem, more than there are workgroups
+ONE = [(1100, 96, 72, 50), (600, 96, 121, 60), (600, 96, 72, 100), (300, 96, 72, 200), (300, 96, 128, 256),
+       (300, 700, 72, 200)]
 # groups of two, three and four workgroups (128, 80 and 64 groups of the 256 resident
-# workgroups), five row blocks and more
-GROUPS = [(160, 160, 40, 300), (160, 200, 96, 300), (100, 160, 128, 600), (80, 161, 121, 900)]
+# workgroups), five row blocks and more; the last as above
+GROUPS = [(160, 160, 40, 300), (160, 200, 96, 300), (100, 160, 128, 600), (80, 161, 121, 900),
+          (149, 1000, 2, 512)]
 
 
 def _stats(hip, x, p):
