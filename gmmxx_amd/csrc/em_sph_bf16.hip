@@ -305,9 +305,7 @@ __global__ __launch_bounds__(64 * NW) void sph_bf16_kernel(TileArgs a) {
         int idx = 0;
         if constexpr (WANT_IDX) idx = group_min_i<NW>((mw == M) ? red_i[o] : 0x7fffffff);
         const int64_t n = n0 + r;
-        if (MODE == MODE_IDX && a.labels) {       // (uniform) every component is in this workgroup
-          if (w == 0 && n < rend) a.labels[(size_t)b * N + n] = (int64_t)idx;
-        } else if (w == 0 && n < rend) {
+        if (w == 0 && n < rend) {
           const size_t og = ((size_t)ktile * a.B + b) * N + n;
           reinterpret_cast<float2*>(a.part_ms)[og] = make_float2(M, t);
           if constexpr (WANT_IDX) a.part_idx[og] = idx;
