@@ -20,9 +20,9 @@
 // its last rounding: of a row that one component dominates the others' share is below half
 // a unit of lse2, and without it every such r is too large, N_k by up to 3e-7).
 //
-// Bound by MFMA and VALU issue, which overlap in part (per wave and block at D = 64:
-// 126 MFMAs, 2016 cycles, beside about 370 VALU instructions; 0.117 ms of MFMA at
-// N = 262144, K = 32).  Statistics launch, fw_stats_kernel -> here: D = 64, K = 32
+// Bound by MFMA and VALU issue, which barely overlap (N = 262144, D = 64, K = 32: busy 44
+// and 46 %; per wave and block 126 MFMAs, 2016 cycles, beside about 370 VALU instructions;
+// 0.117 ms of MFMA).  Statistics launch, fw_stats_kernel -> here: D = 64, K = 32
 // 0.390 -> 0.254 ms; D = 32, K = 32 0.181 -> 0.112; D = 33, K = 32 0.38 -> 0.164;
 // N = 130000: D = 128, K = 16 0.389 -> 0.237; D = 80, K = 24 0.80 -> 0.27.  Error of
 // Σ r x xᵀ against float64 at N = 262144, D = 64, K = 32: 2.6e-7 -> 1.9e-7.

@@ -18,14 +18,14 @@
 // so only one block's exponentials stay in registers (the lag of two of the
 // exchanging kernel, with K in one workgroup, spilled 74 to 120 VGPRs at NW = 8).
 //
-// Bound by VALU issue: per wave and block 163 VALU instructions (21 of them
-// transcendental, none packed) beside 19 MFMAs at D = 128.  One EM iteration
-// against the two passes of em_sph_bf16.hip (which form every logit twice from a
+// Bound by latency: the chain row factors, staging of r, E-GEMM on one accumulator, row
+// maximum, exponentials, barrier at two waves per SIMD (N = 1M, D = 96, K = 200: MFMA busy
+// 23 %, VALU busy 44 %, half of the wave cycles waiting; D = 128, K = 256: 22, 34 and 52 %).
+// One EM iteration against the two passes of em_sph_bf16.hip (which form every logit twice from a
 // hi + lo split, load rows of D != 32, 64, 128 by element, and write and read the
 // row log-normalisers): N = 1M: D = 96, K = 200 0.245 against 0.61 ms; D = 96,
 // K = 50 0.114 / 0.58; D = 100, K = 256 0.26 / 0.60; D = 128, K = 256 0.27 / 0.39;
 // D = 64, K = 128 0.113 / 0.172; N = 50000 x 2, D = 29, K = 100 0.035 / 0.049.
-
 
 #include "common.hpp"
 #include "engine.hpp"
