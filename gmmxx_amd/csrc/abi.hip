@@ -48,6 +48,7 @@ struct Plan {
   int lnw = 0, lktiles = 0;  // waves / component tiles of the plain log-normaliser pass (MODE_LSE)
   bool fused = false;        // EM iteration as one fused pass (small K; em_fused.hip)
   bool sb = false;           // spherical bf16 operands of the single passes and the label pass
+  bool sb_augs = false;      // w_augs among them
   bool coop = false;         // EM iteration as one cooperative pass (spherical bf16; em_coop.hip)
   bool single = false;       // EM iteration as one tile pass (fp32 x, all K in one workgroup; MODE_STATS_LSE)
   bool xch = false;          // EM iteration as one tile pass whose 2..4 component tiles exchange row partials
@@ -226,7 +227,7 @@ int plan_problem(const gmmxx_problem* p, Plan* pl, bool lean = false) {
     const int64_t one = std::min(std::max<int64_t>(1, q.cNG / q.B), most);
     auto cost = [&](int64_t n) { return (q.B * n + q.cNG - 1) / q.cNG * ((row_blocks + n - 1) / n + 4); };
     int64_t spb = one;
-    for (int64_t n = one + 1; n <= std::min(8 * one, most) && q.B > 1; ++n)
+    for (int64_t n = one + 1; !lean && q.B > 1 && n <= std::min(8 * one, most); ++n)
       if (cost(n) < cost(spb) && 10 * cost(n) <= 9 * cost(one)) spb = n;
     // An item is addressed with 32-bit offsets: keep it under 2^30 bytes of x.
     spb = std::max<int64_t>(spb, (q.N * q.DP * 2 + (int64_t(1) << 30) - 1) >> 30);
@@ -314,7 +315,8 @@ int plan_problem(const gmmxx_problem* p, Plan* pl, bool lean = false) {
   q.sb = sph_bf && (lean ? q.coop || q.fused : q.K <= kCoopComps * kMaxCoopGroup);
   q.o_wmu = take(q.sb ? BK * q.DP * 2 : 0);
   q.o_wsc = take(q.sb ? BK * 4 : 0);
-  q.o_waugs = take(q.sb ? BK * 16 * 2 : 0);
+  q.sb_augs = q.sb && !(lean && q.coop);   // (the exchanging pass reads w_aug)
+  q.o_waugs = take(q.sb_augs ? BK * 16 * 2 : 0);
   q.o_cconst = take(BK * 16);
   q.o_covs_used = take(q.cov == SPH ? BK * 4 : (q.cov == DIAG ? BK * q.D * 4 : 0));
   q.o_rowq = take(q.cov == TIED ? BN * 4 : 0);
@@ -633,7 +635,7 @@ int prepare(const Plan& pl, const void* x, const float* means, const float* covs
   a.w_aug = (pl.bf && pl.cov == SPH) ? at<void>(ws, pl.o_waug) : nullptr;
   a.w_mu = pl.sb ? at<void>(ws, pl.o_wmu) : nullptr;
   a.w_scale = pl.sb ? at<float>(ws, pl.o_wsc) : nullptr;
-  a.w_augs = pl.sb ? at<void>(ws, pl.o_waugs) : nullptr;
+  a.w_augs = pl.sb_augs ? at<void>(ws, pl.o_waugs) : nullptr;
   a.cconst = at<float4>(ws, pl.o_cconst);
   a.gram = shift ? gram : nullptr;
   a.shift = gram ? shift : nullptr;

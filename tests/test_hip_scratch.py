@@ -16,6 +16,7 @@ CASES = [  # cov, B, N, D, K, dtype
     ("spherical", 1, 1594715, 88, 47, BF),          # one workgroup per slice: more slices than two passes
     ("spherical", 107, 725, 45, 547, BF),           # groups that exchange: their words and operands
     ("spherical", 127, 54, 108, 236, BF),           # and one-block slices
+    ("spherical", 33, 4354, 128, 562, BF),          # exchanging groups, one item per problem
     ("full", 1, 10535, 75, 94, torch.float32),      # 16-component statistics
 ]
 
